@@ -545,6 +545,57 @@ def _lane_wide_entry():
   return Entry('', [d], F64, {'A': A, 'B': B, 'C': C})
 
 
+def _matrix_entry(kind, m, k, q, fp=F64, beta=None, dense_star=False, mid=0):
+  """Chains with dense shared operands at the edges of the matrix-core forms' row blocks (4, 8 and
+  16 rows), quantity shares and destination placements: ``gemm`` C (+)= A B, ``volume``
+  D (+)= K (Q S), ``chain`` D (+)= V (U (Q S)) with ``mid`` rows between."""
+  pair, ident = [[0, -1], [-1, 1]], [[0, 1], [0, 1]]
+  C = _t([m, q], Addressing.STRIDED, alias='C')
+  A = _t([m, mid or k], Addressing.NONE, alias='A')
+  B = _t([k, q], Addressing.STRIDED, alias='B')
+  tensors = {'A': A, 'B': B, 'C': C}
+  descrs, right = [], _sub(B)
+  if kind != 'gemm':
+    star = None if dense_star else ListSPP([(r, c) for c in range(q) for r in range(q)
+                                            if (r + 2 * c) % 3 == 0], (q, q))
+    S = _t([q, q], Addressing.STRIDED, spp=star, alias='S')
+    tensors['S'] = S
+    T = generate_tmp_tensor([right, _sub(S)], pair)
+    descrs.append(MultilinearDescr(_sub(T), [right, _sub(S)], pair, ident))
+    right = _sub(T)
+  if kind == 'chain':
+    U = _t([mid, k], Addressing.NONE, alias='U')
+    tensors['U'] = U
+    T = generate_tmp_tensor([_sub(U), right], pair)
+    descrs.append(MultilinearDescr(_sub(T), [_sub(U), right], pair, ident))
+    right = _sub(T)
+  descrs.append(GemmDescr(False, False, _sub(A), right, _sub(C), alpha=1.0, beta=beta or 0.0))
+  return Entry('', descrs, fp, tensors)
+
+
+MATRIX_EDGES = {
+  'gemm_5x3': dict(kind='gemm', m=5, k=3, q=9),
+  'gemm_16x16_q1': dict(kind='gemm', m=16, k=16, q=1, beta=1.0),
+  'gemm_18x21_q8': dict(kind='gemm', m=18, k=21, q=8, beta=-0.5),
+  'gemm_33x35_q10': dict(kind='gemm', m=33, k=35, q=10, beta=1.0),
+  'gemm_57x60': dict(kind='gemm', m=57, k=60, q=9, beta=1.0),
+  'gemm_84x83': dict(kind='gemm', m=84, k=83, q=9, beta=1.0),
+  'gemm_7x5_f32': dict(kind='gemm', m=7, k=5, q=9, fp=F32, beta=1.0),
+  'gemm_50x33_q16_f32': dict(kind='gemm', m=50, k=33, q=16, fp=F32),
+  'volume_12': dict(kind='volume', m=12, k=12, q=9, dense_star=True),
+  'volume_35': dict(kind='volume', m=35, k=35, q=9),
+  'volume_41x47_q5': dict(kind='volume', m=41, k=47, q=5, beta=1.0),
+  'volume_90x30_f32': dict(kind='volume', m=90, k=30, q=9, fp=F32),
+  'volume_61x59_f32': dict(kind='volume', m=61, k=59, q=9, fp=F32, beta=2.0, dense_star=True),
+  'volume_84x84': dict(kind='volume', m=84, k=84, q=9, beta=1.0),
+  'chain_56x21x56': dict(kind='chain', m=56, mid=21, k=56, q=9, dense_star=True),
+  'chain_13x6x29_q4': dict(kind='chain', m=13, mid=6, k=29, q=4, beta=1.0),
+  'chain_37x18x50_f32': dict(kind='chain', m=37, mid=18, k=50, q=9, fp=F32, beta=1.0,
+                             dense_star=True),
+}
+for _tag, _kw in MATRIX_EDGES.items():
+  register(f't_matrix_{_tag}_plain')(lambda kw=_kw: _matrix_entry(**kw))
+
 _auto_variants()
 
 

@@ -97,6 +97,10 @@ class Schedule:
   # blocks (prefetch distance = slots - 1)
   stream_dma: bool = False
   stream_dma_slots: int = 3
+  # matrix-core form of the streaming schedule where the chain admits it (dense shared operands):
+  # 'auto' or 'never'. Without an explicit schedule it is the default; the knobs above describe
+  # the vector form, so an explicit schedule keeps that one
+  stream_matrix: str = 'never'
   # how the DPP broadcast is issued: 'asm' (one v_fmac_*_dpp) or 'builtin' (v_mov_*_dpp + fma)
   dpp: str = 'asm'
   # FP64 matrix-core form: wavefronts per workgroup and contraction rows per block (0: chosen
@@ -855,10 +859,14 @@ def starved(emitted) -> bool:
 
 
 def emit(program, context, base_name, schedule=None) -> Emitted:
-  from . import stream
-  schedule = schedule or Schedule()
+  from . import stream, tile
+  schedule = schedule or Schedule(stream_matrix='auto')
   if schedule.stream:
     pl, _ = stream.plan(program)
+    if pl is not None and schedule.stream_matrix == 'auto':
+      emitted, _ = tile.emit(program, context, base_name, pl)
+      if emitted is not None:
+        return emitted
     if pl is not None:
       sched = Schedule(**{**asdict(schedule), 'waves_per_block': schedule.stream_waves,
                           'k_block': schedule.stream_k_block})

@@ -1,0 +1,127 @@
+"""The matrix-core forms of the streaming schedule, on the CPU: row orders, blocks, and which
+calls take the forms.
+
+The index arithmetic of the generated kernels is restated here from the same geometry objects the
+emitter prints, and checked over every chain of ``catalog.MATRIX_EDGES``: each entry the chain needs
+is moved exactly once, nothing outside its window is read, written or multiplied.
+"""
+import pytest
+
+from tensorforge_amd import catalog
+from tensorforge_amd import workloads as W
+from tensorforge_amd.common.basic_types import Addressing, FloatingPointType
+from tensorforge_amd.common.context import Context
+from tensorforge_amd.common.exceptions import GenerationError
+from tensorforge_amd.emit import stream, tile
+from tensorforge_amd.emit.tuned import Schedule
+from tensorforge_amd.generators.generator import Generator
+
+F64, F32 = FloatingPointType.DOUBLE, FloatingPointType.FLOAT
+
+
+def _form(name):
+  e = catalog.get(name)
+  e.generator.generate()
+  program = e.generator.get_program()
+  pl, why = stream.plan(program)
+  assert pl is not None, why
+  from dataclasses import replace
+  pl = replace(pl, terms=[replace(t, L=t.L or pl.L, l_cols=t.l_cols or pl.l_cols)
+                          for t in pl.terms])
+  return e, program, pl
+
+
+@pytest.mark.parametrize('nb', [2, 4])
+@pytest.mark.parametrize('n', list(range(1, 70)) + [83, 84, 120, 128])
+def test_row_order_covers_every_row_once(n, nb):
+  r = tile.Rows(n, nb)
+  rows = [r.row(s, g) for s in range(r.steps) for g in range(4)]
+  assert sorted(x for x in rows if x < n) == list(range(n))
+  assert len(set(rows)) == len(rows) and max(rows) < 4 * r.steps
+  # the C expression agrees, blocks partition the steps, a block's lanes hold adjacent rows
+  for s in range(r.steps):
+    for g in range(4):
+      c = r.row_expr(str(s), str(g)).replace('?', ' and ').replace('/', '//')
+      if '<' in c:
+        cond, rest = c[1:-1].split(' and ', 1)
+        a, b = rest.split(' : ')
+        c = a if eval(cond) else b
+      assert eval(c) == r.row(s, g)
+  assert [s for st, _, k in r.blocks() for s in range(st, st + k)] == list(range(r.steps))
+
+
+@pytest.mark.parametrize('tag', list(catalog.MATRIX_EDGES))
+def test_direct_blocks_read_inside_the_range(tag):
+  e, program, pl = _form(f't_matrix_{tag}_auto')
+  k = tile._Tile(program, e.generator._context, 'x', pl)
+  chosen = k.choose()
+  assert chosen is not None
+  for stages, post, phases, off, wregion in chosen[1]:
+    for ph in phases:
+      n = ph.kr.n
+      for st, base, b in ph.kr.blocks():
+        for g in range(4):
+          sh = max(0, base + b * g - (n - b)) if base + 4 * b > n else 0
+          assert 0 <= base + b * g - sh and base + b * g - sh + b <= n
+          for j in range(b):
+            want = ph.kr.row(st + j, g)
+            assert want == base + b * g + j
+            # the value moved down to step j, or zero past the range
+            assert (want < n) == (sh + j < b)
+    assert off * k.size + tile.WAVES * wregion * k.size <= tile.LDS_LIMIT
+  assert sum(len(h) for h in k.halves) == pl.q
+
+
+def test_forms_by_chain():
+  """Dense shared operands and strided per-element ones take the matrix cores by default; an
+  explicit schedule, sparse or pointer-based operands and fused statements keep their kernels."""
+  def kind(w, fp=F64, **kw):
+    g = Generator(w.descrs, Context('gfx950', 'hip', fp), **kw)
+    g.generate()
+    em = g.get_emitted()
+    return em.schedule.get('matrix')
+  assert kind(W.gemm()) == 'mfma' == kind(W.gemm(F32), F32)
+  assert kind(W.ader_volume(sparse_k=False)) == 'mfma'
+  assert kind(W.ader_volume(F32, sparse_k=False), F32) == 'mfma'
+  assert kind(W.flux_local()) is None and kind(W.ader_derivative(aligned=False)) is None
+  assert kind(W.gemm(), schedule=Schedule()) is None
+  assert kind(W.gemm(), schedule=Schedule(stream_matrix='auto')) == 'mfma'
+  assert kind(W.ader_volume()) is None
+  for name in ('t_gemm_ptr_auto', 't_ab_transb_auto', 't_fused_gemm_pw', 't_five_multiplies_auto'):
+    e = catalog.get(name)
+    e.generator.generate()
+    assert e.generator.get_emitted().schedule.get('matrix') is None
+
+
+def test_in_place_volume_chain_keeps_the_vector_form():
+  """Both quantities' shares of a set are written by different wavefronts: a chain whose
+  destination is its own streamed operand or weight stays on the form that has one."""
+  from tensorforge_amd.common.aux import generate_tmp_tensor
+  from tensorforge_amd.common.matrix.tensor import SubTensor, Tensor
+  from tensorforge_amd.generators.descriptions import MultilinearDescr
+  Q = Tensor([20, 9], Addressing.STRIDED, alias='Q')
+  S = Tensor([9, 9], Addressing.STRIDED, alias='S')
+  K = Tensor([20, 20], Addressing.NONE, alias='K')
+  pair, ident = [[0, -1], [-1, 1]], [[0, 1], [0, 1]]
+  T = generate_tmp_tensor([SubTensor(Q), SubTensor(S)], pair)
+  d = [MultilinearDescr(SubTensor(T), [SubTensor(Q), SubTensor(S)], pair, ident),
+       MultilinearDescr(SubTensor(Q), [SubTensor(K), SubTensor(T)], pair, ident)]
+  g = Generator(d, Context('gfx950', 'hip', F64))
+  g.generate()
+  assert g.get_emitted().schedule.get('matrix') is None
+
+
+def test_grouped_launch_takes_both_forms():
+  """Members in the vector and in the matrix-core form share a workgroup size."""
+  from tensorforge_amd.grouped import GroupedGenerator
+  members = []
+  for w in (W.ader_volume(), W.ader_volume(b=56, sparse_k=False), W.gemm()):
+    g = Generator(w.descrs, Context('gfx950', 'hip', F64))
+    g.generate()
+    members.append(g)
+  grouped = GroupedGenerator(members)
+  try:
+    grouped.generate()
+  except GenerationError as err:
+    pytest.fail(str(err))
+  assert grouped.block == (512, 1, 1)
