@@ -897,12 +897,16 @@ def set_times(program, pl):
   return memory, total * pl.q / 4 / 2200.0
 
 
-def pays(program, pl):
-  """Chains whose matrix time is the longer; a bare product in any case (C += A B, 65,536 elements:
-  208 us in the vector form, 181 here). The others read and write 16 elements in 64-byte pieces,
-  no faster than the vector form (time-derivative step 622 / 617 us, three arrays 293 / 330)."""
+def staged_pays(program, pl):
+  """The staged form moves whole lines but separates a set's steps by barriers: it is the faster
+  one where memory time is the longer and a set is large enough (C += A B over 800 MB: 10 to 84
+  rows 210-295 us against 271-295, flux integral over 131,072 elements 337 against 424); the
+  volume chain has as much matrix time as memory time from 35 rows up and less than 64 KB per set
+  below (35 rows 306 us direct, 399 staged; 20 rows 103 and 134)."""
   memory, matrix = set_times(program, pl)
-  return pl.terms[0].kind == 'global' or matrix >= memory
+  if pl.terms[0].kind == 'global':
+    return True
+  return memory >= matrix and element_traffic(program).per_element * SET >= 64 * 1024
 
 
 def emit(program, context, base_name, pl):
@@ -913,7 +917,9 @@ def emit(program, context, base_name, pl):
   reason = unsupported_reason(program, pl)
   if reason is not None:
     return None, reason
-  if not pays(program, pl):
-    return None, 'memory time is the longer'
-  em = _Tile(program, context, base_name, pl).emit()
+  from .staged import _Staged
+  em = None
+  if staged_pays(program, pl):
+    em = _Staged(program, context, base_name, pl).emit()
+  em = em or _Tile(program, context, base_name, pl).emit()
   return (em, None) if em is not None else (None, 'accumulators or shared operands do not fit')

@@ -1,5 +1,5 @@
-"""The matrix-core forms of the streaming schedule, on the CPU: row orders, blocks, and which
-calls take the forms.
+"""The matrix-core forms of the streaming schedule, on the CPU: row orders, the pieces in which a
+set crosses memory, LDS regions, and which calls take the forms.
 
 The index arithmetic of the generated kernels is restated here from the same geometry objects the
 emitter prints, and checked over every chain of ``catalog.MATRIX_EDGES``: each entry the chain needs
@@ -12,7 +12,7 @@ from tensorforge_amd import workloads as W
 from tensorforge_amd.common.basic_types import Addressing, FloatingPointType
 from tensorforge_amd.common.context import Context
 from tensorforge_amd.common.exceptions import GenerationError
-from tensorforge_amd.emit import stream, tile
+from tensorforge_amd.emit import staged, stream, tile
 from tensorforge_amd.emit.tuned import Schedule
 from tensorforge_amd.generators.generator import Generator
 
@@ -50,6 +50,62 @@ def test_row_order_covers_every_row_once(n, nb):
   assert [s for st, _, k in r.blocks() for s in range(st, st + k)] == list(range(r.steps))
 
 
+def _pieces(p):
+  """[(element, first storage offset, LDS offset, entries moved down)] of every thread's pieces."""
+  out = []
+  for t in range(staged.THREADS):
+    pr = t % p.per_element
+    pm, pp = pr // p.runs, pr % p.runs * p.per
+    e0 = t // p.per_element
+    if e0 >= p.step:
+      continue
+    h = max(0, pp - (p.rows - p.per)) if p.moved else 0
+    for j in range(p.count):
+      e = e0 + j * p.step
+      if e < staged.SET:
+        out.append((e, p.first + pm * p.col_stride + pp - h,
+                    p.lds_base + e * p.lds_elem + pm * p.lds_run + pp, h, pm, pp))
+  return out
+
+
+@pytest.mark.parametrize('tag', list(catalog.MATRIX_EDGES))
+def test_staged_pieces_cover_the_set(tag):
+  e, program, pl = _form(f't_matrix_{tag}_auto')
+  k = staged._Staged(program, e.generator._context, 'x', pl)
+  if not k.prepare():
+    return
+  regions = []
+  for p in k.xstage + [k.out] + [p for _, st in k.wstage for _, _, _, p in st]:
+    got = _pieces(p)
+    seen = {}
+    for el, g, l, h, pm, pp in got:
+      # 16 bytes inside the run, and inside the element's slot
+      run = p.first + pm * p.col_stride
+      assert run <= g and g + p.per <= run + p.rows
+      assert 0 <= g and g + p.per <= p.arg.element_stride
+      assert l % p.per == 0
+      for x in range(p.per):
+        key = (el, pm, pp + x)
+        assert key not in seen
+        seen[key] = g + x + h if pp + x < p.rows else None
+    cols = p.per_element // p.runs
+    for el in range(staged.SET):
+      for m in range(cols):
+        for r in range(p.rows):
+          assert seen[(el, m, r)] == p.first + m * p.col_stride + r
+    regions.append((p, min(l for _, _, l, *_ in got), max(l for _, _, l, *_ in got) + p.per))
+  # LDS: shared entries, then the streamed operand or the results, then the weights
+  shared = sum(s.kr.steps * k.fragment(s.dr) for s in k.stages + k.post)
+  for p, lo, hi in regions:
+    top = k.lds_bytes // k.size if p.lds_base >= k.wbase0 else k.wbase0
+    assert shared <= lo and hi <= top
+  # operand reads and result writes stay inside an element's rows
+  for x, ph in zip(k.xstage, k.phases):
+    assert x.lds_run == 4 * ph.kr.steps and x.lds_run * (x.per_element // x.runs) <= x.lds_elem
+  assert k.out_lds_rows * k.q <= k.out.lds_elem
+  assert k.lds_bytes <= tile.LDS_LIMIT
+
+
 @pytest.mark.parametrize('tag', list(catalog.MATRIX_EDGES))
 def test_direct_blocks_read_inside_the_range(tag):
   e, program, pl = _form(f't_matrix_{tag}_auto')
@@ -79,14 +135,15 @@ def test_forms_by_chain():
     g = Generator(w.descrs, Context('gfx950', 'hip', fp), **kw)
     g.generate()
     em = g.get_emitted()
-    return em.schedule.get('matrix')
-  assert kind(W.gemm()) == 'mfma' == kind(W.gemm(F32), F32)
-  assert kind(W.ader_volume(sparse_k=False)) == 'mfma'
-  assert kind(W.ader_volume(F32, sparse_k=False), F32) == 'mfma'
-  assert kind(W.flux_local()) is None and kind(W.ader_derivative(aligned=False)) is None
-  assert kind(W.gemm(), schedule=Schedule()) is None
-  assert kind(W.gemm(), schedule=Schedule(stream_matrix='auto')) == 'mfma'
-  assert kind(W.ader_volume()) is None
+    return em.schedule.get('matrix'), em.schedule.get('staged', False)
+  assert kind(W.gemm()) == ('mfma', True) == kind(W.gemm(F32), F32)
+  assert kind(W.ader_volume(sparse_k=False)) == ('mfma', False)
+  assert kind(W.ader_volume(F32, sparse_k=False), F32) == ('mfma', False)
+  assert kind(W.flux_local()) == kind(W.flux_neigh()) == ('mfma', True)
+  assert kind(W.ader_derivative(aligned=False)) == ('mfma', True)
+  assert kind(W.gemm(), schedule=Schedule()) == (None, False)
+  assert kind(W.gemm(), schedule=Schedule(stream_matrix='auto')) == ('mfma', True)
+  assert kind(W.ader_volume())[0] is None
   for name in ('t_gemm_ptr_auto', 't_ab_transb_auto', 't_fused_gemm_pw', 't_five_multiplies_auto'):
     e = catalog.get(name)
     e.generator.generate()
@@ -115,7 +172,7 @@ def test_grouped_launch_takes_both_forms():
   """Members in the vector and in the matrix-core form share a workgroup size."""
   from tensorforge_amd.grouped import GroupedGenerator
   members = []
-  for w in (W.ader_volume(), W.ader_volume(b=56, sparse_k=False), W.gemm()):
+  for w in (W.ader_volume(), W.ader_volume(b=20, sparse_k=False), W.gemm()):
     g = Generator(w.descrs, Context('gfx950', 'hip', F64))
     g.generate()
     members.append(g)
