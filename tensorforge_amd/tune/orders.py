@@ -3,8 +3,8 @@
     python -m tensorforge_amd.tune.orders build   --dir D      (CPU: hipcc)
     python -m tensorforge_amd.tune.orders measure --dir D --out F   (GPU)
 
-Every order's chain is built with each candidate streaming schedule (8 wavefronts per workgroup,
-so any choice can join one grouped launch) and timed at its element count in the uneven batch;
+Every order's chain is built with each candidate streaming schedule (the vector form's knobs and
+the matrix-core form; 8 wavefronts per workgroup, so any choice can join one grouped launch) and timed at its element count in the uneven batch;
 the fastest schedule per order is written to ``F`` (JSON). The catalog's grouped entry reads the
 committed choice (``tune/data/mixed_orders_mi355x.json``).
 """
@@ -31,6 +31,7 @@ def candidates():
     out.append({'stream_k_block': kb, 'stream_lds_lookahead': la, 'stream_prefetch': pf})
   for lkb, rows in itertools.product((2, 4, 8), (48, 64, 96)):
     out.append({'stream_loop_k_block': lkb, 'stream_pass_rows': rows})
+  out.append({'stream_matrix': 'auto'})
   return out
 
 
