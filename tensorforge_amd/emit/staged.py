@@ -86,8 +86,8 @@ class _Pieces:
       with w.block(f'if ({self.tag}e + {n * self.step} < {SET})'):
         body(n)
 
-  def at(self, j):
-    return f'bp + {j * self.step * self.arg.element_stride} + {self.tag}g'
+  def at(self, j, bp='bp'):
+    return f'{bp} + {j * self.step * self.arg.element_stride} + {self.tag}g'
 
   def lds(self, j):
     return f'lds + {self.tag}l + {j * self.step * self.lds_elem}'
@@ -361,14 +361,14 @@ class _Staged(_Tile):
     self.w(f'const unsigned live = (unsigned)__ballot(lane < {SET} && set * {SET} + el < numElements '
            '&& (flags == nullptr || fv != 0u));')
 
-  def move(self, x, name, setexpr, first=0):
+  def move(self, x, name, setexpr, first=0, bp='bp'):
     """Registers ``{name}{first + j}`` <- the thread's pieces of array ``x`` of the set. Elements
     past the end of the batch are read as the last one."""
     w = self.w
     vt = self.vec_t[self.per]
     w('{')
     w._depth += 1
-    w(f'const {self.real}* __restrict__ bp = {x.arg.name} + {setexpr} * '
+    w(f'const {self.real}* __restrict__ {bp} = {x.arg.name} + {setexpr} * '
       f'{SET * x.arg.element_stride}ull + {x.arg.name}_extraOffset;')
     w(f'const size_t left = numElements - {setexpr} * {SET};')
     w(f'const int last = left < {SET} ? (int)left - 1 : {SET - 1};')
@@ -377,7 +377,7 @@ class _Staged(_Tile):
     for j in range(x.count):
       with w.block(''):
         w(f'const int past = {x.element(j)} - last;')
-        w(f'{name}{first + j} = __builtin_nontemporal_load(reinterpret_cast<const {vt}*>({x.at(j)} '
+        w(f'{name}{first + j} = __builtin_nontemporal_load(reinterpret_cast<const {vt}*>({x.at(j, bp)} '
           f'- (past > 0 ? past : 0) * {x.arg.element_stride}));')
     w._depth -= 1
     w('}')
@@ -392,7 +392,9 @@ class _Staged(_Tile):
       w(f'{v}[{x}] = {e};')
 
   def fetch(self, pi, setexpr):
-    self.move(self.xstage[pi], 'xv', setexpr)
+    terms = self.phases[pi].terms
+    self.w(f'// rows of term{"" if len(terms) == 1 else "s"} {", ".join(map(str, terms))}')
+    self.move(self.xstage[pi], 'xv', setexpr, bp=f'lp_cur{pi or ""}')
     at = 0
     for _, _, _, p in self.wstage[pi][1]:
       self.move(p, 'wv', setexpr, at)
