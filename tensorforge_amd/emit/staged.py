@@ -589,7 +589,7 @@ class _Staged(_Tile):
               if si == 0:
                 w(f'{real} {t[j]} = {uc(ci, ki)}[{j}] * {v};')
               else:
-                w(f'{t[j]} = __builtin_fma{"" if self.f64 else "f"}({uc(ci, ki)}[{j}], {v}, {t[j]});')
+                w(f'{t[j]} = {self.fp.fma()}({uc(ci, ki)}[{j}], {v}, {t[j]});')
           for j in range(n):
             lim = s.krange[1] - s.k0
             if s.kr.row(st + j, 3) >= lim:

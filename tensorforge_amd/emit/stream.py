@@ -1189,7 +1189,7 @@ class _Stream:
             v = self.fresh('r')
             w(f'{real} {v} = {qv[slots[0][1]]} * {slots[0][0]}_v;')
             for sv, o in slots[1:]:
-              w(f'{v} = __builtin_fma({qv[o]}, {sv}_v, {v});')
+              w(f'{v} = {self.fp.fma()}({qv[o]}, {sv}_v, {v});')
             rv[ti] = v
           else:
             rv[ti] = f'cur{ti}_{j}'
@@ -1392,7 +1392,7 @@ class _Stream:
           v = self.fresh('r')
           w(f'{real} {v} = {qv[slots[0][1]]} * {slots[0][0]}_v;')
           for sv, o in slots[1:]:
-            w(f'{v} = __builtin_fma({qv[o]}, {sv}_v, {v});')
+            w(f'{v} = {self.fp.fma()}({qv[o]}, {sv}_v, {v});')
           rvals[ti] = v
         else:
           rvals[ti] = self.global_rows[bi][(ti, k)]
@@ -1487,7 +1487,7 @@ class _Stream:
           v = self.fresh('r')
           w(f'{real} {v} = {qv[slots[0][1]]} * {slots[0][0]}_v;')
           for sv, o in slots[1:]:
-            w(f'{v} = __builtin_fma({qv[o]}, {sv}_v, {v});')
+            w(f'{v} = {self.fp.fma()}({qv[o]}, {sv}_v, {v});')
           rv[ti] = v
         else:
           rv[ti] = self.global_rows[bi][(ti, k)]
@@ -1534,7 +1534,7 @@ class _Stream:
     else:
       b = self.fresh('bc')
       w(f'const {self.real} {b} = __builtin_amdgcn_mov_dpp({chunk}, {0x150 + lane_in_row}, 0xf, 0xf, true);')
-      w(f'{acc} = __builtin_fma({b}, {r}, {acc});')
+      w(f'{acc} = {self.fp.fma()}({b}, {r}, {acc});')
 
 
 def _row_passes(pl, schedule):

@@ -844,7 +844,7 @@ class _Tile:
         if x == 0:
           w(f'{self.real} {names[j]} = {qv} * {sv};')
         else:
-          w(f'{names[j]} = __builtin_fma{"" if self.f64 else "f"}({qv}, {sv}, {names[j]});')
+          w(f'{names[j]} = {self.fp.fma()}({qv}, {sv}, {names[j]});')
     for j in range(n):
       # rows past this term's own range (a wider term's rows) must not reach the product
       lim = s.krange[1] - s.k0

@@ -445,7 +445,7 @@ class _Emitter:
     a0, v0 = info['terms'][0]
     w(f'{self.real} {v} = lds[{a0} + {info["row0"] + k}] * {v0};')
     for a, vv in info['terms'][1:]:
-      w(f'{v} = __builtin_fma(lds[{a} + {info["row0"] + k}], {vv}, {v});')
+      w(f'{v} = {self.fp.fma()}(lds[{a} + {info["row0"] + k}], {vv}, {v});')
     if info['scale'] is not None:
       w(f'{v} = {info["scale"]} * {v};')
     cache[key] = v
@@ -736,7 +736,7 @@ class _Emitter:
         for _, i, k, val in block:
           r = self.right_value(p, shape, k, cache)
           if r is not None:
-            w(f'{target}[{i}] = __builtin_fma(({self.real}){val}, {r}, {target}[{i}]);')
+            w(f'{target}[{i}] = {self.fp.fma()}(({self.real}){val}, {r}, {target}[{i}]);')
             if i not in touched:
               touched.append(i)
         if self.sched.pin_results:
@@ -764,7 +764,7 @@ class _Emitter:
         for n, (_, i, k, val) in enumerate(chunks[c]):
           r = self.right_value(p, shape, k, cache)
           if r is not None:
-            w(f'{target}[{i}] = __builtin_fma({names[(c, n)]}, {r}, {target}[{i}]);')
+            w(f'{target}[{i}] = {self.fp.fma()}({names[(c, n)]}, {r}, {target}[{i}]);')
       w('__builtin_amdgcn_sched_barrier(0);')
 
   def lds_left(self, p, shape, target):
@@ -809,7 +809,7 @@ class _Emitter:
       for i in range(rows):
         ia = lo0 + i
         for sv in slot_vars:
-          w(f'{target}[{i}] = __builtin_fma({sv}_a[{ia - reg["r0"][0]}], {sv}_v, {target}[{i}]);')
+          w(f'{target}[{i}] = {self.fp.fma()}({sv}_a[{ia - reg["r0"][0]}], {sv}_v, {target}[{i}]);')
       return
     # dense right operand: one LDS read of L(i,k) per term
     cache = {}
@@ -819,7 +819,7 @@ class _Emitter:
         continue
       for i in range(rows):
         ia = lo0 + i
-        w(f'{target}[{i}] = __builtin_fma(({base})[{self._elem_off(reg, shape, ia, k)}], {r}, '
+        w(f'{target}[{i}] = {self.fp.fma()}(({base})[{self._elem_off(reg, shape, ia, k)}], {r}, '
           f'{target}[{i}]);')
 
   def _lds_col_ptr(self, reg, shape, kvar, base):
