@@ -22,11 +22,11 @@ at a time:
 Loads are issued without branches around them and waited for before the results are stored: a
 register written on two paths is copied where they meet, and the memory counter is in order, so
 either mistake turns the requests of the next set into waits (flux integral 428 us with both, 337
-without). Measured, vector form before / this form: C += A B, 56 x 56 by 56 x 9, 65,536 elements FP64
-208 / 139 us (5.7 TB/s); local flux integral, 131,072 elements 468 / 337 us (5.0 TB/s, which is what a
+without; derivative step 659 us with 21 spilled registers, 576 with none). Measured, vector form before / this form: C += A B, 56 x 56 by 56 x 9, 65,536 elements FP64
+208 / 138 us (5.7 TB/s); local flux integral, 131,072 elements 468 / 331 us (5.0 TB/s, which is what a
 plain copy of 56 of every 64 rows reaches); neighbour flux integral, 40,001 elements with a mask
-124 / 116 us; time-derivative step, 131,071 elements 624 / 586 us, three arrays, 50,000 elements
-293 / 277 us (both bound by the steps between the barriers of a set: two wavefronts per SIMD do not
+124 / 116 us; time-derivative step, 131,071 elements 618 / 576 us, three arrays, 50,000 elements
+293 / 252 us (both bound by the steps between the barriers of a set: two wavefronts per SIMD do not
 cover their LDS latencies).
 """
 from typing import Optional
@@ -43,47 +43,80 @@ class _Pieces:
   moves the same piece of elements e0, e0 + step, ...: one offset per thread serves all of them."""
 
   def __init__(self, tag, arg, rows, cols, first, col_stride, lds_rows, lds_elem, lds_base, per,
-               lds_run=None):
-    self.tag, self.arg, self.rows = tag, arg, rows
+               lds_run=None, elements=SET):
+    self.tag, self.arg, self.rows, self.elements = tag, arg, rows, elements
     self.first, self.col_stride = first, col_stride      # storage offset of run 0, of the next run
     self.lds_elem, self.lds_base = lds_elem, lds_base
     self.lds_run = lds_run or lds_rows                   # distance of two runs in LDS
     self.per = per
+    # pieces lie on 16 bytes in LDS
+    self.aligned = self.lds_run % per == 0 and lds_elem % per == 0
     self.runs = lds_rows // per                          # pieces of one run
     self.per_element = self.runs * cols
     self.fits = self.per_element <= THREADS
-    self.count = _ceil(SET, min(SET, max(1, THREADS // self.per_element)))
-    self.step = _ceil(SET, self.count)
+    self.count = _ceil(elements, min(elements, max(1, THREADS // self.per_element)))
+    self.step = _ceil(elements, self.count)
+    # offsets kept in registers over the loop, or formed anew at every use
+    self.held, self.uses = True, 0
     # pieces that pass the end of the run start earlier and are moved down
     self.moved = lds_rows > rows
 
-  def setup(self, w):
+  def declare(self, w):
+    """Before the loop: the thread's offsets where they are held, else its element, run and piece
+    in one register."""
     t = self.tag
-    w(f'int {t}e, {t}g, {t}l{f", {t}h" if self.moved else ""};')
+    w(f'int {t}k;' if not self.held else self.names())
     with w.block(''):
       w(f'const int pr = (int)threadIdx.x % {self.per_element};')
       w(f'const int pm = pr / {self.runs};')
-      w(f'const int pp = (pr - pm * {self.runs}) * {self.per};')
       # threads without a piece: an element past the set (they read the last one's)
-      w(f'{t}e = (int)threadIdx.x / {self.per_element};')
-      w(f'{t}e = {t}e < {self.step} ? {t}e : {SET};')
-      sh = ''
-      if self.moved:
-        w(f'{t}h = pp > {self.rows - self.per} ? pp - {self.rows - self.per} : 0;')
-        sh = f' - {t}h'
-      w(f'{t}g = {t}e * {self.arg.element_stride} + {self.first} + pm * {self.col_stride} + '
-        f'pp{sh};')
-      w(f'{t}l = {self.lds_base} + {t}e * {self.lds_elem} + pm * {self.lds_run} + pp;')
+      w(f'const int pt = (int)threadIdx.x / {self.per_element};')
+      w(f'const int pe = pt < {self.step} ? pt : {self.elements};')
+      if self.held:
+        w(f'const int pp = (pr - pm * {self.runs}) * {self.per};')
+        self.offsets(w)
+      else:
+        w(f'{t}k = pe << 20 | pm << 12 | (pr - pm * {self.runs});')
+
+  def setup(self, w):
+    """The offsets, at a use."""
+    if self.held:
+      return
+    t = self.tag
+    w(self.names())
+    with w.block(''):
+      w(f'int pk = {t}k;')
+      # may be scheduled freely, but neither leaves the loop nor serves another use as well
+      self.uses += 1
+      w(f'asm("; {t} {self.uses}" : "+v"(pk) : "s"((unsigned)set));')
+      w('const int pe = pk >> 20;')
+      w('const int pm = pk >> 12 & 255;')
+      w(f'const int pp = (pk & 4095) * {self.per};')
+      self.offsets(w)
+
+  def names(self):
+    t = self.tag
+    return f'int {t}e, {t}g, {t}l{f", {t}h" if self.moved else ""};'
+
+  def offsets(self, w):
+    t = self.tag
+    w(f'{t}e = pe;')
+    sh = ''
+    if self.moved:
+      w(f'{t}h = pp > {self.rows - self.per} ? pp - {self.rows - self.per} : 0;')
+      sh = f' - {t}h'
+    w(f'{t}g = {t}e * {self.arg.element_stride} + {self.first} + pm * {self.col_stride} + pp{sh};')
+    w(f'{t}l = {self.lds_base} + {t}e * {self.lds_elem} + pm * {self.lds_run} + pp;')
 
   def each(self, w, body):
     """``body(j)`` for every piece of the thread that exists."""
-    even = self.step * self.count == SET
+    even = self.step * self.count == self.elements
     n = self.count if even else self.count - 1
-    with w.block(f'if ({self.tag}e < {SET})'):
+    with w.block(f'if ({self.tag}e < {self.elements})'):
       for j in range(n):
         body(j)
     if not even:
-      with w.block(f'if ({self.tag}e + {n * self.step} < {SET})'):
+      with w.block(f'if ({self.tag}e + {n * self.step} < {self.elements})'):
         body(n)
 
   def at(self, j, bp='bp'):
@@ -96,7 +129,225 @@ class _Pieces:
     return f'({self.tag}e + {j * self.step})'
 
 
-class _Staged(_Tile):
+class _SetKernel:
+  """A workgroup's loop over sets of ``elements`` elements: the way of the operands and results
+  between memory, registers and LDS. A form supplies its geometry (``xstage`` and ``wstage`` per
+  phase, ``out``, ``dest``, ``old_early``) and ``shared``, ``acc_declare``, ``compute``, ``results``."""
+
+  def barrier(self):
+    # this wavefront's LDS accesses done, every wavefront here; memory accesses stay in flight
+    self.w('asm volatile("s_waitcnt lgkmcnt(0)\\n\\ts_barrier" ::: "memory");')
+
+  def body(self):
+    w = self.w
+    self.shared()
+    for x in self.xstage:
+      x.declare(w)
+    for _, stage in self.wstage:
+      for _, _, _, p in stage:
+        p.declare(w)
+    self.out.declare(w)
+    w(f'const size_t nsets = (numElements + {self.elements - 1}) / {self.elements};')
+    beta = self.beta_load()
+    vt = self.lds_t
+    n = max(x.count for x in self.xstage)
+    w(f'{vt} {", ".join(f"xv{j}" for j in range(n))};')
+    nw = max((sum(p.count for _, _, _, p in st) for _, st in self.wstage), default=0)
+    if nw:
+      w(f'{vt} {", ".join(f"wv{j}" for j in range(nw))};')
+    if beta is not None:
+      w(f'{vt} {", ".join(f"dv{j}" for j in range(self.out.count))};')
+    touches = []
+    if beta is not None and not self.old_early:
+      touches = [f'touched{j}' for j in range(self.touches())]
+      w(f'unsigned {", ".join(touches)};')
+    w('size_t set = blockIdx.x;')
+    self.fetch(0, 'set')
+    self.arrived()
+    with w.block('for (; set < nsets; set += gridDim.x)'):
+      self.acc_declare()
+      for pi, ph in enumerate(self.phases):
+        self.put(pi)
+        self.barrier()
+        last = pi == len(self.phases) - 1
+        if last:
+          self.mask_load()
+          if beta is not None and self.old_early:
+            self.move(self.out, 'dv', 'set')
+          elif beta is not None:
+            self.touch()
+          with w.block('if (set + gridDim.x < nsets)'):
+            self.fetch(0, '(set + gridDim.x)')
+        else:
+          self.fetch(pi + 1, 'set')
+        self.compute(pi)
+        self.barrier()
+      self.results()
+      self.barrier()
+      if touches:
+        w(f'asm volatile("" :: {", ".join(f"{chr(34)}v{chr(34)}({t})" for t in touches)});')
+        self.move(self.out, 'dv', 'set')
+      # the next set's operands have arrived before the results are stored: waiting for them
+      # afterwards would wait for the stores as well
+      self.arrived()
+      self.leave(beta)
+      self.barrier()
+
+  # ------------------------------------------------------------------ memory <-> registers <-> LDS
+  def arrived(self):
+    """Waits for the registers of the first phase's operands."""
+    held = [f'xv{j}' for j in range(self.xstage[0].count)]
+    held += [f'wv{j}' for j in range(sum(p.count for _, _, _, p in self.wstage[0][1]))]
+    for j in range(0, len(held), 8):
+      self.w(f'asm volatile("" : {", ".join(f"{chr(34)}+v{chr(34)}({v})" for v in held[j:j + 8])});')
+
+  def touch(self):
+    """One load per 128-byte line of the old destination: the lines come into the L2 while the
+    products run."""
+    w = self.w
+    o = self.out
+    per = 128 // self.size
+    end = o.first + (self.q - 1) * o.col_stride + o.rows        # of an element's window
+    w('{')
+    w._depth += 1
+    w(f'const size_t left = numElements - set * {self.elements};')
+    w(f'const int last = ((left < {self.elements} ? (int)left : {self.elements}) - 1) * '
+      f'{o.arg.element_stride} + {end - 1};')
+    w(f'const {self.real}* __restrict__ bp = {o.arg.name} + set * '
+      f'{self.elements * o.arg.element_stride}ull + {o.arg.name}_extraOffset;')
+    for j in range(self.touches()):
+      w(f'const int line{j} = {o.first} + ((int)threadIdx.x + {j * THREADS}) * {per};')
+      w(f'touched{j} = *reinterpret_cast<const unsigned*>(bp + (line{j} < last ? line{j} : last));')
+    w._depth -= 1
+    w('}')
+
+  def touches(self):
+    return _ceil(self.elements * self.dest.element_stride, 128 // self.size * THREADS)
+
+  def mask_load(self):
+    """The element's flag, requested early. Without flags the load reads the destination."""
+    w = self.w
+    e = f'set * {self.elements} + lane'
+    w(f'const size_t ef = {e} < numElements ? {e} : numElements - 1;')
+    w(f'const unsigned fv = *(flags != nullptr ? flags + ef : reinterpret_cast<const unsigned*>('
+      f'{self.dest.name} + ef * {self.dest.element_stride}ull + {self.dest.name}_extraOffset));')
+
+  def mask(self):
+    """Bit e: element e of the set is to be stored."""
+    self.w(f'const unsigned long long live = __ballot(lane < {self.elements} && '
+           f'set * {self.elements} + lane < numElements && (flags == nullptr || fv != 0u));')
+
+  def move(self, x, name, setexpr, first=0, bp='bp'):
+    """Registers ``{name}{first + j}`` <- the thread's pieces of array ``x`` of the set. Elements
+    past the end of the batch are read as the last one."""
+    w = self.w
+    vt = self.vec_t[self.per]
+    w('{')
+    w._depth += 1
+    w(f'const {self.real}* __restrict__ {bp} = {x.arg.name} + {setexpr} * '
+      f'{self.elements * x.arg.element_stride}ull + {x.arg.name}_extraOffset;')
+    w(f'const size_t left = numElements - {setexpr} * {self.elements};')
+    w(f'const int last = left < {self.elements} ? (int)left - 1 : {self.elements - 1};')
+    x.setup(w)
+    # no branch around a load: its register would be copied where the paths meet, and the copy
+    # would wait for the load
+    for j in range(x.count):
+      with w.block(''):
+        w(f'const int past = {x.element(j)} - last;')
+        w(f'{name}{first + j} = __builtin_nontemporal_load(reinterpret_cast<const {vt}*>('
+          f'{x.at(j, bp)} - (past > 0 ? past : 0) * {x.arg.element_stride}));')
+    w._depth -= 1
+    w('}')
+
+  def moved_down(self, v, h):
+    """Entries of a piece that was read ``h`` entries early, zeros past the end."""
+    w = self.w
+    for x in range(self.per):
+      e = f'({self.real})0'
+      for d in range(self.per - 1 - x, -1, -1):
+        e = f'({h} == {d} ? {v}[{x + d}] : {e})'
+      w(f'{v}[{x}] = {e};')
+
+  def fetch(self, pi, setexpr):
+    terms = self.phases[pi].terms
+    self.w(f'// rows of term{"" if len(terms) == 1 else "s"} {", ".join(map(str, terms))}')
+    self.move(self.xstage[pi], 'xv', setexpr, bp=f'lp_cur{pi or ""}')
+    at = 0
+    for _, _, _, p in self.wstage[pi][1]:
+      self.move(p, 'wv', setexpr, at)
+      at += p.count
+
+  def put(self, pi):
+    """The phase's operands from registers into LDS."""
+    w = self.w
+    at = 0
+    for p, name in [(self.xstage[pi], 'xv')] + [(p, 'wv') for _, _, _, p in self.wstage[pi][1]]:
+      first = at if name == 'wv' else 0
+
+      def store(j):
+        v = f'{name}{first + j}'
+        if p.moved:
+          self.moved_down(v, f'{p.tag}h')
+        if p.aligned:
+          w(f'*reinterpret_cast<{self.lds_t}*>({p.lds(j)}) = {v};')
+        else:
+          for x in range(self.per):
+            w(f'({p.lds(j)})[{x}] = {v}[{x}];')
+      with w.block(''):
+        p.setup(w)
+        p.each(w, store)
+      at += p.count if name == 'wv' else 0
+
+  def leave(self, beta):
+    """The results from LDS into the destination, the old one added; whole sets without a mask
+    take the first branch."""
+    w = self.w
+    o = self.out
+    vt = self.vec_t[self.per]
+    o.setup(w)
+    scale = '' if beta in (None, 1.0) else f'{self.fp.literal(beta)} * '
+    w(f'{self.real}* __restrict__ bp = {o.arg.name} + set * '
+      f'{self.elements * o.arg.element_stride}ull + {o.arg.name}_extraOffset;')
+
+    def write(j):
+      if o.aligned:
+        w(f'{self.lds_t} rv = *reinterpret_cast<const {self.lds_t}*>({o.lds(j)});')
+      else:
+        w(f'{self.lds_t} rv = {{{", ".join(f"({o.lds(j)})[{x}]" for x in range(self.per))}}};')
+      if beta is not None:
+        if o.moved:
+          self.moved_down(f'dv{j}', 'dh')
+        w(f'rv = {scale}dv{j} + rv;')
+      full = f'__builtin_nontemporal_store(({vt})rv, reinterpret_cast<{vt}*>({o.at(j)}));'
+      if not o.moved:
+        w(full)
+        return
+      with w.block('if (dh == 0)'):
+        w(full)
+      with w.block('else'):
+        for x in range(o.rows % o.per):
+          w(f'({o.at(j)})[dh + {x}] = rv[{x}];')
+
+    def masked(j):
+      with w.block(f'if (live >> {o.element(j)} & 1ull)'):
+        write(j)
+
+    def scoped(body):
+      def run(j):
+        with w.block(''):
+          body(j)
+      return run
+
+    self.mask()
+    with w.block(f'if (live == {(1 << self.elements) - 1}ull)'):
+      o.each(w, scoped(write))
+    with w.block('else'):
+      o.each(w, scoped(masked))
+
+
+class _Staged(_SetKernel, _Tile):
+  elements = SET
+
   def prepare(self):
     """Geometry; False when the chain does not fit this form."""
     pl = self.pl
@@ -183,6 +434,14 @@ class _Staged(_Tile):
     self.old_early = use + old <= 256
     if self.old_early:
       use += old
+    # three or four registers per array: with up to three arrays all offsets stay, with more of them
+    # those of the destination (they are needed at once, between two barriers) unless several
+    # streamed operands take turns. What does not fit is spilled, and a spilled register's reload
+    # waits for every load in flight (derivative step 131,071 elements, all held 659 us, none 606,
+    # the destination's 578; three arrays, 50,000 elements, 278 / 252 / 259 us; flux integral, three
+    # arrays here, all 331 us, none 345)
+    for p in pieces:
+      p.held = len(pieces) <= 3 or (p is self.out and len(self.phases) == 1)
     self.weights_held = 2 if use + slots <= 256 else 1
     return use <= 256
 
@@ -252,11 +511,8 @@ class _Staged(_Tile):
                    extra_launch_setup=persistent_grid(self.kname, self.lds_bytes, THREADS, SET,
                                                       f'launcher_{self.base_name}'))
 
-  def barrier(self):
-    # this wavefront's LDS accesses done, every wavefront here; memory accesses stay in flight
-    self.w('asm volatile("s_waitcnt lgkmcnt(0)\\n\\ts_barrier" ::: "memory");')
-
-  def body(self):
+  def shared(self):
+    """The shared operands into LDS, and the lane's place."""
     w = self.w
     real = self.real
     w(f'extern __shared__ __align__(16) {real} lds[];')
@@ -269,193 +525,6 @@ class _Staged(_Tile):
     w('const int g = lane / 16;')
     w(f'const {real}* __restrict__ ka = ubuf + lane;')
     w(f'const {real}* __restrict__ ks = ubuf + (lane % 4 + 4 * g);')
-    w(f'const size_t nsets = (numElements + {SET - 1}) / {SET};')
-    for x in self.xstage:
-      x.setup(w)
-    for _, stage in self.wstage:
-      for _, _, _, p in stage:
-        p.setup(w)
-    self.out.setup(w)
-    beta = self.beta_load()
-    vt = self.lds_t
-    n = max(x.count for x in self.xstage)
-    w(f'{vt} {", ".join(f"xv{j}" for j in range(n))};')
-    nw = max((sum(p.count for _, _, _, p in st) for _, st in self.wstage), default=0)
-    if nw:
-      w(f'{vt} {", ".join(f"wv{j}" for j in range(nw))};')
-    if beta is not None:
-      w(f'{vt} {", ".join(f"dv{j}" for j in range(self.out.count))};')
-    touches = []
-    if beta is not None and not self.old_early:
-      touches = [f'touched{j}' for j in range(_ceil(SET * self.dest.element_stride,
-                                                    128 // self.size * THREADS))]
-      w(f'unsigned {", ".join(touches)};')
-    w('size_t set = blockIdx.x;')
-    self.fetch(0, 'set')
-    self.arrived()
-    with w.block('for (; set < nsets; set += gridDim.x)'):
-      self.acc_declare()
-      for pi, ph in enumerate(self.phases):
-        self.put(pi)
-        self.barrier()
-        last = pi == len(self.phases) - 1
-        if last:
-          self.mask_load()
-          if beta is not None and self.old_early:
-            self.move(self.out, 'dv', 'set')
-          elif beta is not None:
-            self.touch()
-          with w.block('if (set + gridDim.x < nsets)'):
-            self.fetch(0, '(set + gridDim.x)')
-        else:
-          self.fetch(pi + 1, 'set')
-        self.compute(pi)
-        self.barrier()
-      self.results()
-      self.barrier()
-      if touches:
-        w(f'asm volatile("" :: {", ".join(f"{chr(34)}v{chr(34)}({t})" for t in touches)});')
-        self.move(self.out, 'dv', 'set')
-      # the next set's operands have arrived before the results are stored: waiting for them
-      # afterwards would wait for the stores as well
-      self.arrived()
-      self.leave(beta)
-      self.barrier()
-
-  # ------------------------------------------------------------------ memory <-> registers <-> LDS
-  def arrived(self):
-    """Waits for the registers of the first phase's operands."""
-    held = [f'xv{j}' for j in range(self.xstage[0].count)]
-    held += [f'wv{j}' for j in range(sum(p.count for _, _, _, p in self.wstage[0][1]))]
-    for j in range(0, len(held), 8):
-      self.w(f'asm volatile("" : {", ".join(f"{chr(34)}+v{chr(34)}({v})" for v in held[j:j + 8])});')
-
-  def touch(self):
-    """One load per 128-byte line of the old destination: the lines come into the L2 while the
-    products run."""
-    w = self.w
-    d = self.dest
-    per = 128 // self.size
-    total = SET * d.element_stride
-    w('{')
-    w._depth += 1
-    w(f'const size_t entries = (numElements - set * {SET} < {SET} ? numElements - set * {SET} : '
-      f'{SET}) * {d.element_stride}ull;')
-    w(f'const {self.real}* __restrict__ bp = {d.name} + set * {total}ull + {d.name}_extraOffset;')
-    for j in range(_ceil(total, per * THREADS)):
-      w(f'const size_t line{j} = ((size_t)threadIdx.x + {j * THREADS}) * {per};')
-      w(f'touched{j} = *reinterpret_cast<const unsigned*>(bp + (line{j} < entries ? line{j} : '
-        'entries - 1));')
-    w._depth -= 1
-    w('}')
-
-  def mask_load(self):
-    """The element's flag, requested early. Without flags the load reads the destination."""
-    w = self.w
-    w(f'const size_t ef = set * {SET} + el < numElements ? set * {SET} + el : numElements - 1;')
-    w(f'const unsigned fv = *(flags != nullptr ? flags + ef : reinterpret_cast<const unsigned*>('
-      f'{self.dest.name} + ef * {self.dest.element_stride}ull + {self.dest.name}_extraOffset));')
-
-  def mask(self):
-    """Bit e: element e of the set is to be stored."""
-    self.w(f'const unsigned live = (unsigned)__ballot(lane < {SET} && set * {SET} + el < numElements '
-           '&& (flags == nullptr || fv != 0u));')
-
-  def move(self, x, name, setexpr, first=0, bp='bp'):
-    """Registers ``{name}{first + j}`` <- the thread's pieces of array ``x`` of the set. Elements
-    past the end of the batch are read as the last one."""
-    w = self.w
-    vt = self.vec_t[self.per]
-    w('{')
-    w._depth += 1
-    w(f'const {self.real}* __restrict__ {bp} = {x.arg.name} + {setexpr} * '
-      f'{SET * x.arg.element_stride}ull + {x.arg.name}_extraOffset;')
-    w(f'const size_t left = numElements - {setexpr} * {SET};')
-    w(f'const int last = left < {SET} ? (int)left - 1 : {SET - 1};')
-    # no branch around a load: its register would be copied where the paths meet, and the copy
-    # would wait for the load
-    for j in range(x.count):
-      with w.block(''):
-        w(f'const int past = {x.element(j)} - last;')
-        w(f'{name}{first + j} = __builtin_nontemporal_load(reinterpret_cast<const {vt}*>({x.at(j, bp)} '
-          f'- (past > 0 ? past : 0) * {x.arg.element_stride}));')
-    w._depth -= 1
-    w('}')
-
-  def moved_down(self, v, h):
-    """Entries of a piece that was read ``h`` entries early, zeros past the end."""
-    w = self.w
-    for x in range(self.per):
-      e = f'({self.real})0'
-      for d in range(self.per - 1 - x, -1, -1):
-        e = f'({h} == {d} ? {v}[{x + d}] : {e})'
-      w(f'{v}[{x}] = {e};')
-
-  def fetch(self, pi, setexpr):
-    terms = self.phases[pi].terms
-    self.w(f'// rows of term{"" if len(terms) == 1 else "s"} {", ".join(map(str, terms))}')
-    self.move(self.xstage[pi], 'xv', setexpr, bp=f'lp_cur{pi or ""}')
-    at = 0
-    for _, _, _, p in self.wstage[pi][1]:
-      self.move(p, 'wv', setexpr, at)
-      at += p.count
-
-  def put(self, pi):
-    """The phase's operands from registers into LDS."""
-    w = self.w
-    at = 0
-    for p, name in [(self.xstage[pi], 'xv')] + [(p, 'wv') for _, _, _, p in self.wstage[pi][1]]:
-      first = at if name == 'wv' else 0
-
-      def store(j):
-        v = f'{name}{first + j}'
-        if p.moved:
-          self.moved_down(v, f'{p.tag}h')
-        w(f'*reinterpret_cast<{self.lds_t}*>({p.lds(j)}) = {v};')
-      p.each(w, store)
-      at += p.count if name == 'wv' else 0
-
-  def leave(self, beta):
-    """The results from LDS into the destination, the old one added; whole sets without a mask
-    take the first branch."""
-    w = self.w
-    o = self.out
-    vt = self.vec_t[self.per]
-    scale = '' if beta in (None, 1.0) else f'{self.fp.literal(beta)} * '
-    w(f'{self.real}* __restrict__ bp = {o.arg.name} + set * {SET * o.arg.element_stride}ull + '
-      f'{o.arg.name}_extraOffset;')
-
-    def write(j):
-      w(f'{self.lds_t} rv = *reinterpret_cast<const {self.lds_t}*>({o.lds(j)});')
-      if beta is not None:
-        if o.moved:
-          self.moved_down(f'dv{j}', 'dh')
-        w(f'rv = {scale}dv{j} + rv;')
-      full = f'__builtin_nontemporal_store(({vt})rv, reinterpret_cast<{vt}*>({o.at(j)}));'
-      if not o.moved:
-        w(full)
-        return
-      with w.block('if (dh == 0)'):
-        w(full)
-      with w.block('else'):
-        for x in range(o.rows % o.per):
-          w(f'({o.at(j)})[dh + {x}] = rv[{x}];')
-
-    def masked(j):
-      with w.block(f'if (live >> {o.element(j)} & 1u)'):
-        write(j)
-
-    def scoped(body):
-      def run(j):
-        with w.block(''):
-          body(j)
-      return run
-
-    self.mask()
-    with w.block(f'if (live == {(1 << SET) - 1}u)'):
-      o.each(w, scoped(write))
-    with w.block('else'):
-      o.each(w, scoped(masked))
 
   # ------------------------------------------------------------------ products
   def columns(self):
