@@ -79,6 +79,64 @@ class Writer:
     return '\n'.join(self._lines) + '\n'
 
 
+FILL_LOADS = 8
+
+
+def fill_shared(w, total, threads, steps, put):
+  """Copies ``total`` shared entries into LDS, entry ``e = threadIdx.x + i * threads`` by each
+  thread. ``steps``: [(type, name, lines, value)], the loads of one entry, each allowed to use the
+  names of earlier ones; ``put(e, v)``: the store.
+
+  The loads of up to FILL_LOADS entries are written side by side, without branches (threads past
+  the end read the last entry again): as one loop over the entries each iteration waits for its
+  own loads: 8 iterations of two dependent loads for the 3,715 entries of the sparse volume chain
+  (100 elements FP64 31.1 us so, 29.9 now), 19 of one for the dense chain of 56 rows (65,536
+  elements FP64 213 / 206 us; 100,003 FP32 187 / 179), 42 for 84 rows (30,000 elements 254 / 235),
+  500,000 elements of orders 2..7 1,169 / 1,140."""
+  if total == 0:
+    return
+  n = (total + threads - 1) // threads
+  batches = (n + FILL_LOADS - 1) // FILL_LOADS
+  b = (n + batches - 1) // batches
+  last = f'const int e = eb + i * {threads} < {total} ? eb + i * {threads} : {total - 1};'
+  with w.block(f'for (int eb = threadIdx.x; eb < {batches * b * threads}; eb += {b * threads})'):
+    for t, name, _, _ in steps:
+      w(f'{t} {name}s[{b}];')
+    for k, (t, name, lines, value) in enumerate(steps):
+      w('#pragma unroll')
+      with w.block(f'for (int i = 0; i < {b}; ++i)'):
+        w(last)
+        for t0, name0, _, _ in steps[:k]:
+          w(f'const {t0} {name0} = {name0}s[i];')
+        for line in lines:
+          w(line)
+        w(f'{name}s[i] = {value};')
+    w('#pragma unroll')
+    with w.block(f'for (int i = 0; i < {b}; ++i)'):
+      # the last entry again, with its own value: a condition would draw the load behind it
+      w(last)
+      w(f'{put("e", f"{steps[-1][1]}s[i]")};')
+
+
+def fill_from_table(w, total, threads, real, table, shared, put):
+  """:func:`fill_shared` for entries of several operands at the positions a table lists (operand
+  in the bits from 20 on)."""
+  names = [f.arg.name for f in shared]
+  lines = ['const unsigned t = tv >> 20;', 'const unsigned pos = tv & 0xfffffu;']
+  if len({f.arg.dtype for f in shared}) == 1:
+    # one load: an operand chosen by the loaded value would be a branch around each load
+    pick = names[-1]
+    for i in range(len(names) - 2, -1, -1):
+      pick = f'(t == {i} ? {names[i]} : {pick})'
+    value = f'({real}){pick}[pos]'
+  else:
+    value = f'({real}){names[-1]}[pos]'
+    for i in range(len(names) - 2, -1, -1):
+      value = f'(t == {i} ? ({real}){names[i]}[pos] : {value})'
+  fill_shared(w, total, threads,
+              [('unsigned', 'tv', [], f'{table}[e]'), (real, 'uv', lines, value)], put)
+
+
 def kernel_params(program, context):
   """Parameter list of the ``__global__`` kernel: the launcher's, minus ``streamPtr``."""
   params = []

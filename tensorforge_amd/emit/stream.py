@@ -25,7 +25,7 @@ from typing import List, Optional
 from ..common.basic_types import Addressing, FloatingPointType
 from ..common.exceptions import GenerationError
 from . import ir
-from .launcher import Emitted, Writer, kernel_params, persistent_grid
+from .launcher import Emitted, Writer, fill_from_table, fill_shared, kernel_params, persistent_grid
 from .traffic import element_traffic
 
 WAVE = 64
@@ -458,35 +458,29 @@ class _Stream:
     w(f'const int col = lane / {q} < {G} ? lane - slot * {q} : 0;')
     # stage the shared entries
     if not self.loop:
-      with w.block(f'for (int e = threadIdx.x; e < {self.nu}; e += {threads})'):
-        w(f'const unsigned tv = {self.utab}[e];')
-        w('const unsigned t = tv >> 20;')
-        w('const unsigned pos = tv & 0xfffffu;')
-        shared = [t.U for t in pl.terms] + [st.U for st in pl.post]
-        expr = f'({real}){shared[-1].arg.name}[pos]'
-        for t_idx in range(len(shared) - 2, -1, -1):
-          expr = f'(t == {t_idx} ? ({real}){shared[t_idx].arg.name}[pos] : {expr})'
+      def put(e, v):
         if self.pair:
           # chunk pairs interleaved: entry j of chunks 2c and 2c + 1 side by side
-          w(f'ubuf[((e >> 5) << 5) | ((e & 15) << 1) | ((e >> 4) & 1)] = {expr};')
-        else:
-          w(f'ubuf[e] = {expr};')
+          return f'ubuf[(({e} >> 5) << 5) | (({e} & 15) << 1) | (({e} >> 4) & 1)] = {v}'
+        return f'ubuf[{e}] = {v}'
+      fill_from_table(w, self.nu, threads, real, self.utab,
+                      [t.U for t in pl.terms] + [st.U for st in pl.post], put)
     elif self.u_source == 'lds':
       nt = len(pl.terms)
       rp = self.rows_pad
       nrows = pl.rows[1] - pl.rows[0]
-      with w.block(f'for (int e = threadIdx.x; e < {self.nu_pad}; e += {threads})'):
-        w(f'const int i = e % {rp};')
-        w(f'const int t = (e / {rp}) % {nt};')
-        w(f'const int k = e / {rp * nt} + {pl.klo};')
-        expr = self.lit(0)
-        for t_idx in range(nt - 1, -1, -1):
-          U = pl.terms[t_idx].U
-          nd, kd = pl.terms[t_idx].u_dims
-          pos = (f'(i + {pl.rows[0] - U.origin[nd]}) * {U.strides[nd]} + (k - {U.origin[kd]}) * '
-                 f'{U.strides[kd]}')
-          expr = f'(t == {t_idx} ? ({real}){U.arg.name}[{pos}] : {expr})'
-        w(f'ubuf[e] = i < {nrows} ? {expr} : {self.lit(0)};')
+      lines = [f'const int ri = e % {rp};', f'const int t = (e / {rp}) % {nt};',
+               f'const int k = e / {rp * nt} + {pl.klo};']
+      expr = self.lit(0)
+      for t_idx in range(nt - 1, -1, -1):
+        U = pl.terms[t_idx].U
+        nd, kd = pl.terms[t_idx].u_dims
+        pos = (f'(ri + {pl.rows[0] - U.origin[nd]}) * {U.strides[nd]} + (k - {U.origin[kd]}) * '
+               f'{U.strides[kd]}')
+        expr = f'(t == {t_idx} ? ({real}){U.arg.name}[{pos}] : {expr})'
+      fill_shared(w, self.nu_pad, threads,
+                  [(real, 'uv', lines, f'ri < {nrows} ? {expr} : {self.lit(0)}')],
+                  lambda e, v: f'ubuf[{e}] = {v}')
     w('__syncthreads();')
     self.per_lane_setup()
     w(f'const size_t ngroups = (numElements + {G - 1}) / {G};')

@@ -31,8 +31,8 @@ What bounds it: FP64 matrix instructions and FP64 FMAs share one unit (measured 
 1.09 + 1.31 ms, 2.46 ms), 70-75 TF for either; the vector form's DPP-broadcast FMA reaches 49-58 TF
 at its two wavefronts per SIMD and pays for the address of every lane's own cache line. FP32 matrix
 instructions run at 125-150 TF beside the vector unit. Measured on MI355X, vector form before / this
-form: order-6 volume chain with dense K_d, 65,536 elements FP64 335 / 213 us (55 TF), 100,003
-elements FP32 409 / 187 us (95 TF); order 7, 30,000 elements FP64 432 / 254 us. Matrix instructions
+form: order-6 volume chain with dense K_d, 65,536 elements FP64 335 / 206 us (57 TF), 100,003
+elements FP32 409 / 179 us (99 TF); order 7, 30,000 elements FP64 432 / 235 us. Matrix instructions
 are issued 62 % of the cycles there, the FP64 FMAs of the temporaries take another 5 %; fragments
 read further ahead, the next term's temporaries formed among the matrix instructions, or rows
 shared through LDS (a barrier per block) did not change or lost time.
@@ -42,7 +42,7 @@ from typing import List, Optional
 
 from ..common.basic_types import Addressing, FloatingPointType
 from . import ir
-from .launcher import Emitted, Writer, kernel_params, persistent_grid
+from .launcher import Emitted, Writer, fill_shared, kernel_params, persistent_grid
 from .traffic import element_traffic
 
 WAVE = 64
@@ -103,6 +103,12 @@ class Rows:
     f = self.full * self.nb
     return (f'(({step}) < {f} ? {body} : {self.full * 4 * self.nb} + {self.tail} * ({g}) + '
             f'({step}) - {f})')
+
+  def row_sum(self, step, g):
+    """:meth:`row_expr` with one choice between constants, for code that must not branch."""
+    n = self.nb if not self.tail else \
+        f'({step} < {self.full * self.nb} ? {self.nb} : {self.tail})'
+    return f'{step} / {self.nb} * {4 * self.nb} + {n} * {g} + {step} % {self.nb}'
 
 
 @dataclass
@@ -393,32 +399,30 @@ class _Tile:
     total = s.kr.steps * F
     if total == 0:
       return
-    with w.block(f'for (int e = threadIdx.x; e < {total}; e += {WAVE * WAVES})'):
-      w(f'const int st = e / {F};')
-      w(f'const int f = e - st * {F};')
-      pick = lambda a, b: a if not small else (b if not big else f'(f < {64 * big} ? {a} : {b})')
-      if self.f64:
-        w(f'const int j = {pick("f / 64 * 4 + f % 16 / 4", f"{4 * big} + (f - {64 * big}) / 16")};')
-        w(f'const int g = {pick("f % 4", "f % 4")};')
-        w(f'const int kg = {pick("f % 64 / 16", f"(f - {64 * big}) % 16 / 4")};')
-      else:
-        w('const int j = f / 64 * 4 + f % 4;')
-        w('const int g = f % 16 / 4;')
-        w('const int kg = f % 64 / 16;')
-      w(f'const int row = {self.row_of(s.dr, "j", "g")};')
-      w(f'const int k = {s.kr.row_expr("st", "kg")} + {s.k0};')
-      w(f'const bool in = row >= 0 && row < {nrows} && k >= {s.krange[0]} && k < {s.krange[1]};')
-      pos = (f'(row + {s.rows[0] - s.U.origin[nd]}) * {s.U.strides[nd]} + (k - {s.U.origin[kd]}) * '
-             f'{s.U.strides[kd]}')
-      w(f'ubuf[{s.base} + e] = in ? {s.U.arg.name}[in ? {pos} : 0] : ({self.real})0;')
-
-  def row_of(self, dr, j, g):
-    """Destination row of result register ``j`` (run-time). FP32 tiles have four registers; those
-    past the last block's steps hold no row."""
-    e = dr.row_expr(j, g)
-    if self.f64 or dr.steps % 4 == 0:
-      return e
-    return f'(({j}) < {dr.steps} ? {e} : -1)'
+    # every value on a line of its own: a conditional expression of such terms becomes a branch,
+    # and a branch between two entries keeps their loads apart
+    lines = [f'const int st = e / {F};', f'const int f = e - st * {F};']
+    if self.f64:
+      # 16-row tiles, then 4-row tiles
+      lines += ['const int j1 = f / 64 * 4 + f % 16 / 4;', 'const int kg1 = f % 64 / 16;',
+                f'const int j2 = {4 * big} + (f - {64 * big}) / 16;',
+                f'const int kg2 = (f - {64 * big}) % 16 / 4;',
+                f'const int j = f < {64 * big} ? j1 : j2;',
+                f'const int kg = f < {64 * big} ? kg1 : kg2;', 'const int g = f % 4;']
+    else:
+      lines += ['const int j = f / 64 * 4 + f % 4;', 'const int g = f % 16 / 4;',
+                'const int kg = f % 64 / 16;']
+    # FP32 tiles have four registers; those past the last block's steps hold no row
+    lines += [f'const int row = {s.dr.row_sum("j", "g")};',
+              f'const int k = {s.kr.row_sum("st", "kg")} + {s.k0};',
+              f'const bool in = (j < {s.dr.steps}) & (row < {nrows}) & (k >= {s.krange[0]}) & '
+              f'(k < {s.krange[1]});',
+              f'const int pos = (row + {s.rows[0] - s.U.origin[nd]}) * {s.U.strides[nd]} + '
+              f'(k - {s.U.origin[kd]}) * {s.U.strides[kd]};',
+              f'const {self.real} u = {s.U.arg.name}[in ? pos : 0];']
+    fill_shared(w, total, WAVE * WAVES,
+                [(self.real, 'uv', lines, f'in ? u : ({self.real})0')],
+                lambda e, v: f'ubuf[{s.base} + {e}] = {v}')
 
   def band(self, window, plan):
     w = self.w
