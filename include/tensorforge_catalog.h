@@ -57,6 +57,20 @@ void launcher_kernel_9ebda1b851(double* m0, unsigned m0_extraOffset, const doubl
 void launcher_kernel_2304a85efa(float* m0, unsigned m0_extraOffset, const float* m1, unsigned m1_extraOffset, const float* m2, unsigned m2_extraOffset, float m3, size_t numElements, unsigned* flags, void* streamPtr);
 /* t_dense_sparse_auto, t_dense_sparse_plain */
 void launcher_kernel_54b5fd2a96(double* m0, unsigned m0_extraOffset, const double* m1, unsigned m1_extraOffset, const double* m2, size_t numElements, unsigned* flags, void* streamPtr);
+/* t_few_gemm_41x38_auto, t_few_gemm_41x38_plain */
+void launcher_kernel_5b78b5f2a0(double* m0, unsigned m0_extraOffset, const double* m1, const double* m2, unsigned m2_extraOffset, size_t numElements, unsigned* flags, void* streamPtr);
+/* t_few_gemm_70x30_q13_f32_auto, t_few_gemm_70x30_q13_f32_plain */
+void launcher_kernel_e68807b4c9(float* m0, unsigned m0_extraOffset, const float* m1, const float* m2, unsigned m2_extraOffset, size_t numElements, unsigned* flags, void* streamPtr);
+/* t_few_gemm_9x4_q1_auto, t_few_gemm_9x4_q1_plain */
+void launcher_kernel_4c6db7f131(double* m0, unsigned m0_extraOffset, const double* m1, const double* m2, unsigned m2_extraOffset, size_t numElements, unsigned* flags, void* streamPtr);
+/* t_few_volume_10_auto, t_few_volume_10_plain */
+void launcher_kernel_a4ac5f0ee0(const double* m0, unsigned m0_extraOffset, const double* m1, unsigned m1_extraOffset, double* m2, unsigned m2_extraOffset, const double* m3, size_t numElements, unsigned* flags, void* streamPtr);
+/* t_few_volume_35x29_q6_auto, t_few_volume_35x29_q6_plain */
+void launcher_kernel_4ad28f7e1c(const double* m0, unsigned m0_extraOffset, const double* m1, unsigned m1_extraOffset, double* m2, unsigned m2_extraOffset, const double* m3, size_t numElements, unsigned* flags, void* streamPtr);
+/* t_few_volume_57x58_f32_auto, t_few_volume_57x58_f32_plain */
+void launcher_kernel_97f4bb87ef(const float* m0, unsigned m0_extraOffset, const float* m1, unsigned m1_extraOffset, float* m2, unsigned m2_extraOffset, const float* m3, size_t numElements, unsigned* flags, void* streamPtr);
+/* t_few_volume_83x84_f32_auto, t_few_volume_83x84_f32_plain */
+void launcher_kernel_bafcf4791a(const float* m0, unsigned m0_extraOffset, const float* m1, unsigned m1_extraOffset, float* m2, unsigned m2_extraOffset, const float* m3, size_t numElements, unsigned* flags, void* streamPtr);
 /* t_five_multiplies_auto, t_five_multiplies_plain */
 void launcher_kernel_b3ac723cd6(const float* m0, unsigned m0_extraOffset, const float* m1, unsigned m1_extraOffset, const float* m2, unsigned m2_extraOffset, float* m3, unsigned m3_extraOffset, const float* m4, unsigned m4_extraOffset, size_t numElements, unsigned* flags, void* streamPtr);
 /* t_four_matrices_auto, t_four_matrices_plain */

@@ -545,13 +545,16 @@ def _lane_wide_entry():
   return Entry('', [d], F64, {'A': A, 'B': B, 'C': C})
 
 
-def _matrix_entry(kind, m, k, q, fp=F64, beta=None, dense_star=False, mid=0):
+def _matrix_entry(kind, m, k, q, fp=F64, beta=None, dense_star=False, mid=0, sparse=False):
   """Chains with dense shared operands at the edges of the matrix-core forms' row blocks (4, 8 and
   16 rows), quantity shares and destination placements: ``gemm`` C (+)= A B, ``volume``
-  D (+)= K (Q S), ``chain`` D (+)= V (U (Q S)) with ``mid`` rows between."""
+  D (+)= K (Q S), ``chain`` D (+)= V (U (Q S)) with ``mid`` rows between. ``sparse``: a pattern of
+  two fifths in the shared operand."""
   pair, ident = [[0, -1], [-1, 1]], [[0, 1], [0, 1]]
   C = _t([m, q], Addressing.STRIDED, alias='C')
-  A = _t([m, mid or k], Addressing.NONE, alias='A')
+  mask = ListSPP([(r, c) for c in range(k) for r in range(m) if (2 * r + 3 * c) % 5 < 2],
+                 (m, k)) if sparse else None
+  A = _t([m, mid or k], Addressing.NONE, spp=mask, alias='A')
   B = _t([k, q], Addressing.STRIDED, alias='B')
   tensors = {'A': A, 'B': B, 'C': C}
   descrs, right = [], _sub(B)
@@ -595,6 +598,20 @@ MATRIX_EDGES = {
 }
 for _tag, _kw in MATRIX_EDGES.items():
   register(f't_matrix_{_tag}_plain')(lambda kw=_kw: _matrix_entry(**kw))
+
+# sparse shared operands at the edges of the form for few elements: rows and contraction rows per
+# wavefront (4), entries per table batch, columns per wavefront (64)
+FEW_EDGES = {
+  'gemm_9x4_q1': dict(kind='gemm', m=9, k=4, q=1, beta=1.0),
+  'gemm_41x38': dict(kind='gemm', m=41, k=38, q=9),
+  'gemm_70x30_q13_f32': dict(kind='gemm', m=70, k=30, q=13, fp=F32, beta=1.0),
+  'volume_10': dict(kind='volume', m=10, k=10, q=9),
+  'volume_35x29_q6': dict(kind='volume', m=35, k=29, q=6, beta=-0.5),
+  'volume_57x58_f32': dict(kind='volume', m=57, k=58, q=9, fp=F32, beta=2.0, dense_star=True),
+  'volume_83x84_f32': dict(kind='volume', m=83, k=84, q=9, fp=F32),
+}
+for _tag, _kw in FEW_EDGES.items():
+  register(f't_few_{_tag}_plain')(lambda kw=_kw: _matrix_entry(sparse=True, **kw))
 
 _auto_variants()
 

@@ -36,9 +36,12 @@ class Emitted:
   # launcher's parameters) is false
   fallback: 'Emitted' = None
   condition: str = ''
+  # a kernel of the same chain for launches of at most ``few_limit`` elements
+  few: 'Emitted' = None
+  few_limit: int = 0
 
   def full_source(self):
-    return self.kernel_src + (self.fallback.full_source() if self.fallback else '')
+    return self.kernel_src + ''.join(e.full_source() for e in (self.fallback, self.few) if e)
 
 
 class Writer:
@@ -172,6 +175,10 @@ def launcher_source(generator, emitted: Emitted) -> str:
     w(f'if ({GeneralLexicon.NUM_ELEMENTS} == 0) return;')
     w(f'hipStream_t stream = ({GeneralLexicon.STREAM_PTR_STR} != nullptr) ? '
       f'static_cast<hipStream_t>({GeneralLexicon.STREAM_PTR_STR}) : 0;')
+    if emitted.few is not None:
+      with w.block(f'if ({GeneralLexicon.NUM_ELEMENTS} <= {emitted.few_limit})'):
+        _launch_block(w, generator, emitted.few)
+        w('return;')
     if emitted.fallback is not None:
       with w.block(f'if ({emitted.condition})'):
         _launch_block(w, generator, emitted)
@@ -261,11 +268,12 @@ def distinct_symbol(emitted: Emitted) -> Emitted:
   new = f'{old}_{form}_{digest}'
 
   def rename(em):
-    fb = rename(em.fallback) if em.fallback is not None else None
+    fb, few = (rename(e) if e is not None else None for e in (em.fallback, em.few))
     return dataclasses.replace(em, kernel_name=em.kernel_name.replace(old, new),
                                kernel_src=em.kernel_src.replace(old, new),
                                extra_launch_setup=em.extra_launch_setup.replace(old, new),
-                               condition=em.condition.replace(old, new), fallback=fb)
+                               condition=em.condition.replace(old, new), fallback=fb,
+                               few=few)
   return rename(emitted)
 
 

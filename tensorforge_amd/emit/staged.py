@@ -43,7 +43,7 @@ class _Pieces:
   moves the same piece of elements e0, e0 + step, ...: one offset per thread serves all of them."""
 
   def __init__(self, tag, arg, rows, cols, first, col_stride, lds_rows, lds_elem, lds_base, per,
-               lds_run=None, elements=SET):
+               lds_run=None, elements=SET, threads=THREADS):
     self.tag, self.arg, self.rows, self.elements = tag, arg, rows, elements
     self.first, self.col_stride = first, col_stride      # storage offset of run 0, of the next run
     self.lds_elem, self.lds_base = lds_elem, lds_base
@@ -53,8 +53,8 @@ class _Pieces:
     self.aligned = self.lds_run % per == 0 and lds_elem % per == 0
     self.runs = lds_rows // per                          # pieces of one run
     self.per_element = self.runs * cols
-    self.fits = self.per_element <= THREADS
-    self.count = _ceil(elements, min(elements, max(1, THREADS // self.per_element)))
+    self.fits = self.per_element <= threads
+    self.count = _ceil(elements, min(elements, max(1, threads // self.per_element)))
     self.step = _ceil(elements, self.count)
     # offsets kept in registers over the loop, or formed anew at every use
     self.held, self.uses = True, 0
@@ -132,7 +132,8 @@ class _Pieces:
 class _SetKernel:
   """A workgroup's loop over sets of ``elements`` elements: the way of the operands and results
   between memory, registers and LDS. A form supplies its geometry (``xstage`` and ``wstage`` per
-  phase, ``out``, ``dest``, ``old_early``) and ``shared``, ``acc_declare``, ``compute``, ``results``."""
+  phase, ``out``, ``dest``, ``old_early``) and ``place``, ``shared``, ``acc_declare``, ``compute``,
+  ``results``."""
 
   def barrier(self):
     # this wavefront's LDS accesses done, every wavefront here; memory accesses stay in flight
@@ -140,7 +141,7 @@ class _SetKernel:
 
   def body(self):
     w = self.w
-    self.shared()
+    self.place()
     for x in self.xstage:
       x.declare(w)
     for _, stage in self.wstage:
@@ -162,7 +163,9 @@ class _SetKernel:
       touches = [f'touched{j}' for j in range(self.touches())]
       w(f'unsigned {", ".join(touches)};')
     w('size_t set = blockIdx.x;')
+    # the first set's operands are on their way while the shared ones are staged
     self.fetch(0, 'set')
+    self.shared()
     self.arrived()
     with w.block('for (; set < nsets; set += gridDim.x)'):
       self.acc_declare()
@@ -511,20 +514,21 @@ class _Staged(_SetKernel, _Tile):
                    extra_launch_setup=persistent_grid(self.kname, self.lds_bytes, THREADS, SET,
                                                       f'launcher_{self.base_name}'))
 
-  def shared(self):
-    """The shared operands into LDS, and the lane's place."""
+  def place(self):
     w = self.w
     real = self.real
     w(f'extern __shared__ __align__(16) {real} lds[];')
     w(f'{real}* __restrict__ ubuf = lds;')
-    for s in self.stages + self.post:
-      self.stage_shared(s)
     w(f'const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / {WAVE});')
     w(f'const int lane = threadIdx.x % {WAVE};')
     w('const int el = lane % 16;')
     w('const int g = lane / 16;')
     w(f'const {real}* __restrict__ ka = ubuf + lane;')
     w(f'const {real}* __restrict__ ks = ubuf + (lane % 4 + 4 * g);')
+
+  def shared(self):
+    for s in self.stages + self.post:
+      self.stage_shared(s)
 
   # ------------------------------------------------------------------ products
   def columns(self):

@@ -134,7 +134,8 @@ class Phase:
   kr: Rows
 
 
-def unsupported_reason(program, pl):
+def set_unsupported_reason(program, pl):
+  """Why whole elements of a chain cannot be staged in LDS, or None."""
   if program.epilogue is not None:
     return 'pointwise statements fused into the chain'
   kinds = {t.kind for t in pl.terms}
@@ -144,10 +145,6 @@ def unsupported_reason(program, pl):
     return 'a per-element operand is not strided'
   if any(a.kind != ir.SRC_GLOBAL or a.dtype != program.fp_type for a in program.args):
     return 'an operand by value or of another type'
-  if pl.q > 16:
-    return 'more than 16 columns'
-  if any(t.U.is_sparse() for t in pl.terms) or any(s.U.is_sparse() for s in pl.post):
-    return 'sparse shared operand'
   if pl.dest_product.dest_strides[0] != 1:
     return 'destination rows are not contiguous'
   final = pl.post[-1].product if pl.post else pl.dest_product
@@ -159,7 +156,7 @@ def unsupported_reason(program, pl):
     if t.kind == 'fused':
       if t.L.arg is pl.dest:
         return 'the destination is also the streamed operand'
-      if t.L.strides[0] != 1 or t.l_cols[1] - t.l_cols[0] > 16:
+      if t.L.strides[0] != 1:
         return 'streamed operand layout'
       if t.W.arg is pl.dest:
         return 'the destination is also a weight'
@@ -169,6 +166,14 @@ def unsupported_reason(program, pl):
       if t.B.arg is pl.dest and len(pl.terms) > 1:
         return 'the destination is also an operand'
   return None
+
+
+def unsupported_reason(program, pl):
+  if pl.q > 16 or any(t.kind == 'fused' and t.l_cols[1] - t.l_cols[0] > 16 for t in pl.terms):
+    return 'more than 16 columns'
+  if any(t.U.is_sparse() for t in pl.terms) or any(s.U.is_sparse() for s in pl.post):
+    return 'sparse shared operand'
+  return set_unsupported_reason(program, pl)
 
 
 class _Tile:

@@ -859,7 +859,7 @@ def starved(emitted) -> bool:
 
 
 def emit(program, context, base_name, schedule=None) -> Emitted:
-  from . import stream, tile
+  from . import small, stream, tile
   schedule = schedule or Schedule(stream_matrix='auto')
   if schedule.stream:
     pl, _ = stream.plan(program)
@@ -872,6 +872,9 @@ def emit(program, context, base_name, schedule=None) -> Emitted:
                           'k_block': schedule.stream_k_block})
       emitted = stream.emit(program, context, base_name, sched, pl)
       if emitted.lds_bytes <= LDS_LIMIT:
+        if schedule.stream_matrix == 'auto':
+          emitted.few = small.emit(program, context, base_name, sched, pl)
+          emitted.few_limit = small.limit(emitted.few) if emitted.few else 0
         return emitted
   if program.epilogue is not None:
     raise GenerationError('pointwise statements fuse only into a streaming chain')
