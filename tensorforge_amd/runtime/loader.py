@@ -68,6 +68,7 @@ class Kernel:
       raise RuntimeError(f'{self.name} is not exported by {lib._name}') from err
     self.signature = generator.launcher_signature()
     self.fn.argtypes = [_ctype(t) for t, _ in self.signature]
+    self.pointers = [i for i, (t, _) in enumerate(self.signature) if t.endswith('*')]
     self.fn.restype = None
     self.lib = lib
 
@@ -75,13 +76,13 @@ class Kernel:
     if len(args) != len(self.signature):
       raise TypeError(f'{self.name} takes {len(self.signature)} arguments '
                       f'({", ".join(n for _, n in self.signature)}), given {len(args)}')
-    conv = []
-    for (t, _), a in zip(self.signature, args):
-      if t.endswith('*'):
-        conv.append(None if a is None or a == 0 else ctypes.c_void_p(int(a)))
-      else:
-        conv.append(a)
-    self.fn(*conv)
+    if any(type(args[i]) is not int for i in self.pointers):
+      args = list(args)
+      for i in self.pointers:
+        a = args[i]
+        args[i] = None if a is None or a == 0 else ctypes.c_void_p(int(a))
+    # ctypes passes ints as the pointers the prototype declares
+    self.fn(*args)
     err = runtime().tensorforge_last_error()
     if err != 0:
       where = runtime().tensorforge_last_error_where().decode()
