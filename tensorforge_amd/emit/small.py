@@ -48,6 +48,8 @@ class _Phase:
 
 
 class _Small(_SetKernel):
+  shared_last = False
+
   def __init__(self, program, context, base_name, schedule, pl):
     self.prog, self.ctx, self.pl = program, context, pl
     self.base_name = base_name

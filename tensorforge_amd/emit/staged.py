@@ -14,8 +14,10 @@ at a time:
 3. each of the eight wavefronts forms the products of its own quantity (B operands are one 16-byte
    LDS read per streamed column and block; elements are 16 bytes off a multiple of the bank period,
    so 16 lanes reading the same row of 16 elements meet no conflict). A ninth quantity is divided
-   among the wavefronts by row tiles, so that every SIMD does the same work; further ones go to one
-   wavefront each;
+   so that every SIMD does the same work: its contraction among four wavefronts, each forming the
+   temporaries of its own blocks only (derivative step, 131,071 elements: 549 us; divided by row
+   tiles, with the temporaries of all rows in each of three wavefronts, 576). Further quantities go
+   to one wavefront each;
 4. the results replace the streamed operand in LDS and leave as a linear run, with the old
    destination added.
 
@@ -25,7 +27,7 @@ either mistake turns the requests of the next set into waits (flux integral 428 
 without; derivative step 659 us with 21 spilled registers, 576 with none). Measured, vector form before / this form: C += A B, 56 x 56 by 56 x 9, 65,536 elements FP64
 208 / 138 us (5.7 TB/s); local flux integral, 131,072 elements 468 / 331 us (5.0 TB/s, which is what a
 plain copy of 56 of every 64 rows reaches); neighbour flux integral, 40,001 elements with a mask
-124 / 116 us; time-derivative step, 131,071 elements 618 / 576 us, three arrays, 50,000 elements
+124 / 116 us; time-derivative step, 131,071 elements 618 / 549 us, three arrays, 50,000 elements
 293 / 252 us (both bound by the steps between the barriers of a set: two wavefronts per SIMD do not
 cover their LDS latencies).
 """
@@ -36,6 +38,7 @@ from .tile import LDS_LIMIT, SET, WAVE, WAVES, _ceil, _Tile
 from .traffic import element_traffic
 
 THREADS = WAVE * WAVES
+SHARES = 4                    # wavefronts that divide a ninth quantity, one on each SIMD
 
 
 class _Pieces:
@@ -312,11 +315,22 @@ class _SetKernel:
     w(f'{self.real}* __restrict__ bp = {o.arg.name} + set * '
       f'{self.elements * o.arg.element_stride}ull + {o.arg.name}_extraOffset;')
 
+    if self.shared_last:
+      # the thread's place in the other shares of the last quantity
+      w(f'const int sl = dl - {o.lds_base + (self.q - 1) * o.lds_run} - de * {o.lds_elem};')
+      w(f'const {self.real}* sp = lds + {self.share_base} + de * {self.share_elem} + sl;')
+
     def write(j):
       if o.aligned:
         w(f'{self.lds_t} rv = *reinterpret_cast<const {self.lds_t}*>({o.lds(j)});')
       else:
         w(f'{self.lds_t} rv = {{{", ".join(f"({o.lds(j)})[{x}]" for x in range(self.per))}}};')
+      if self.shared_last:
+        # (all of them before the first is added: 29 spilled registers, 582 us against 549)
+        with w.block('if (sl >= 0)'):
+          for i in range(SHARES - 1):
+            w(f'rv += *reinterpret_cast<const {self.lds_t}*>(sp + '
+              f'{(j * o.step + i * SET) * self.share_elem});')
       if beta is not None:
         if o.moved:
           self.moved_down(f'dv{j}', 'dh')
@@ -415,18 +429,26 @@ class _Staged(_SetKernel, _Tile):
     # against 295 in the direct form; 56 x 13: 319 against 268)
     if self.lds_bytes > LDS_LIMIT or not all(p.fits and p.count <= 8 for p in pieces):
       return False
-    # a wavefront's quantities: its own, and a share of the ninth (row tiles) or one more
+    # a wavefront's quantities: its own and one more, or a share of the ninth: SHARES wavefronts
+    # divide its contraction, their sums meet in LDS in place of the weights or behind them
     self.extra = max(0, self.q - WAVES)
-    big, small = self.tiles(dr)
-    cols = 1 if self.extra == 0 or (self.extra == 1 and not self.post) else 2
-    self.divided = self.extra == 1 and not self.post
+    self.share_base, self.share_elem = wbase, skew(lds_rows, 256 // self.size)
+    end = max(wbase + wsize, wbase + (SHARES - 1) * SET * self.share_elem) * self.size
+    self.shared_last = self.extra == 1 and not self.post and self.fused and end <= LDS_LIMIT
+    # a bare product waits for memory: its ninth quantity is divided by row tiles, which adds
+    # nothing to the way of the results (138 us; in shares of the contraction 142)
+    self.tiled_last = self.extra == 1 and not self.post and not self.fused
+    if self.shared_last:
+      self.lds_bytes = max(self.lds_bytes, end)
+    cols = 1 if self.extra == 0 or self.shared_last or self.tiled_last else 2
     acc = max((4 * self.tiles(s.dr)[0] + self.tiles(s.dr)[1]) for s in self.stages + self.post)
-    acc = acc * cols + (4 if self.divided else 0)
+    # the share's accumulators beside the own ones only over several phases
+    acc = acc * (2 if self.shared_last and len(self.phases) > 1 else cols) + 4 * self.tiled_last
     # registers (32-bit): accumulators, operands on the way, streamed rows, weights
     words = self.size // 4
     held = 4 * (max(x.count for x in self.xstage) +
                 max((sum(p.count for _, _, _, p in st) for _, st in self.wstage), default=0))
-    reads = max(sum(4 if len(set(k)) == 1 else 4 * cols + 4 * self.divided
+    reads = max(sum(4 if len(set(k)) == 1 else 4 * cols + 4 * self.tiled_last
                     for k in self.keys(ph)) for ph in self.phases)
     slots = max(sum(len(self.slots(ti)) for ti in ph.terms) for ph in self.phases) * words \
         if self.fused else 0
@@ -537,14 +559,13 @@ class _Staged(_SetKernel, _Tile):
     own = ('acc', 'wave', None)
     if self.q < WAVES:
       return [(f'wave < {self.q}', [own])]
-    if not self.extra:
+    if not self.extra or self.shared_last:
       return [('', [own])]
-    if not self.divided:
+    if not self.tiled_last:
       return [(f'wave < {self.extra}', [own, ('acx', f'(wave + {WAVES})', None)]), ('', [own])]
-    dr = self.last.dr
-    big, small = self.tiles(dr)
+    big, small = self.tiles(self.last.dr)
     # 16-row tiles made of whole blocks are alike: tile ``wave``; the others together
-    uniform = big if self.f64 else dr.full
+    uniform = big if self.f64 else self.last.dr.full
     out = []
     if uniform:
       out.append((f'wave < {uniform}', [own, ('acu', str(WAVES), ('u',))]))
@@ -556,25 +577,20 @@ class _Staged(_SetKernel, _Tile):
 
   def acc_declare(self):
     """Accumulators of every variant (a wavefront uses its own), cleared."""
-    w = self.w
     first = self.stages[0].dr
-    zero = f'({self.real})0'
     names = {n for _, cols in self.columns() for n, _, _ in cols}
+    if self.shared_last:
+      names.add('acx')
     for n in ('acc', 'acx'):
       if n in names:
         self.declare_acc(n, first, [0])
-        if self.post:
-          for i, s in enumerate(self.post):
-            self.declare_acc(f'{n}p{i}', s.dr, [0])
-    self.acc_big['acr'] = self.acc_big['acc']
+        for i, s in enumerate(self.post):
+          self.declare_acc(f'{n}p{i}', s.dr, [0])
     if 'acu' in names:
-      w(f'{self.acc_t} acu_0_0 = {{{zero}, {zero}, {zero}, {zero}}};')
+      self.declare_acc('acu', first, [0], ((0,), ()))
     if 'acr' in names:
-      big, small = next(t for _, cols in self.columns() for n, _, t in cols if n == 'acr')[1:]
-      for t in big:
-        w(f'{self.acc_t} acr_0_{t} = {{{zero}, {zero}, {zero}, {zero}}};')
-      for i in small:
-        w(f'{self.real} acr_0s{i} = {zero};')
+      tiles = next(t for _, cols in self.columns() for n, _, t in cols if n == 'acr')
+      self.declare_acc('acr', first, [0], tiles[1:])
 
   def variants(self, emit):
     w = self.w
@@ -585,6 +601,55 @@ class _Staged(_SetKernel, _Tile):
 
   def compute(self, pi):
     self.variants(lambda cols: self.compute_columns(pi, cols))
+    if self.shared_last:
+      with self.w.block(f'if (wave < {SHARES})'):
+        self.compute_share(pi)
+
+  def compute_share(self, pi):
+    """The wavefront's blocks of the last quantity's contraction, every fourth one."""
+    w, real, ph = self.w, self.real, self.phases[pi]
+    x, c = self.xstage[pi], self.q - 1
+    welem, wst = self.wstage[pi]
+    keys = self.keys(ph)
+    col0 = ph.cols[0] if ph.cols is not None else 0
+    w(f'const {real}* __restrict__ xb = lds + {x.lds_base} + el * {x.lds_elem};')
+    w(f'const {real}* __restrict__ wb = lds + {self.wbase0} + el * {welem};')
+    offs = {ti: off - lo for ti, lo, off, _ in wst}
+
+    def block(st, base, n):
+      for ki, m in enumerate(keys):
+        at = f'xb + {(m[c] - col0) * x.lds_run} + {base} + {n} * g'
+        if n == self.per:
+          w(f'const {self.lds_t} u{ki} = *reinterpret_cast<const {self.lds_t}*>({at});')
+        else:
+          w(f'{self.lds_t} u{ki} = {{{", ".join(f"({at})[{j}]" for j in range(n))}}};')
+      for ti in ph.terms:
+        s = self.stages[ti]
+        ops = []
+        for j in range(n):
+          t, first = self.fresh('xt'), True
+          for m, p in self.slots(ti) if self.fused else ():
+            if p[c] < 0:
+              continue
+            v, u = f'wb[{offs[ti] + p[c]}]', f'u{keys.index(m)}[{j}]'
+            w(f'{real} {t} = {u} * {v};' if first else f'{t} = {self.fp.fma()}({u}, {v}, {t});')
+            first = False
+          if first:
+            w(f'{real} {t} = {f"({real})0" if self.fused else f"u0[{j}]"};')
+          lim = s.krange[1] - s.k0
+          if self.fused and lim < 4 * ph.kr.steps:
+            # rows past this term's own range must not reach the product
+            w(f'{t} = {base} + {j} + {n} * g < {lim} ? {t} : ({real})0;')
+          ops.append(t)
+        for j in range(n):
+          self.step(s, f'{s.base} + ({st} + {j}) * {self.fragment(s.dr)}', [('acx', str(c), None)], [ops[j]])
+
+    if ph.kr.full:
+      with w.block(f'for (int b = wave; b < {ph.kr.full}; b += {SHARES})'):
+        block(f'b * {self.nb}', f'b * {4 * self.nb}', self.nb)
+    if ph.kr.tail:
+      with w.block(f'if (wave == {ph.kr.full % SHARES})'):
+        block(ph.kr.full * self.nb, ph.kr.full * 4 * self.nb, ph.kr.tail)
 
   def compute_columns(self, pi, cols):
     w = self.w
@@ -705,11 +770,9 @@ class _Staged(_SetKernel, _Tile):
     for t in range(big):
       a = self.fresh('xa')
       w(f'const {self.real} {a} = ka[{off} + {64 * t}];')
-      for name, op in whole:
+      for name, op in whole + [(nm, op) for nm, tiles, op in rest
+                               if tiles[0] == 'r' and t in tiles[1]]:
         w(f'{name}_0_{t} = {fn}({a}, {op}, {name}_0_{t}, 0, 0, 0);')
-      for name, tiles, op in rest:
-        if tiles[0] == 'r' and t in tiles[1]:
-          w(f'{name}_0_{t} = {fn}({a}, {op}, {name}_0_{t}, 0, 0, 0);')
     for i in range(small):
       a = self.fresh('xa')
       w(f'const {self.real} {a} = ks[{off} + {64 * big + 16 * i}];')
@@ -724,33 +787,45 @@ class _Staged(_SetKernel, _Tile):
 
   # ------------------------------------------------------------------ results
   def results(self):
-    self.variants(self.result_columns)
+    w, o = self.w, self.out
+    ob = f'{self.real}* __restrict__ ob = lds + {o.lds_base} + el * {o.lds_elem}'
 
-  def result_columns(self, cols):
+    def columns(cols):
+      w(f'{ob};')
+      for name, c, tiles in cols:
+        self.result_column(name, f'{c} * {self.out_lds_rows}', tiles)
+    self.variants(columns)
+    if self.shared_last:
+      with w.block(f'if (wave < {SHARES})'):
+        # the first share in its place, the others to be added to it
+        w(f'{ob};')
+        w(f'const int at = wave == 0 ? {(self.q - 1) * o.lds_run} : {self.share_base - o.lds_base} + '
+          f'((wave - 1) * {SET} + el) * {self.share_elem} - el * {o.lds_elem};')
+        self.result_column('acx', 'at')
+
+  def result_column(self, name, at, tiles=None):
     w = self.w
     dr = self.last.dr
-    w(f'{self.real}* __restrict__ ob = lds + {self.out.lds_base} + el * {self.out.lds_elem};')
-    big, small = self.tiles(dr)
-    for name, c, tiles in cols:
-      if self.post:
-        name = f'{name}p{len(self.post) - 1}'
-      if tiles is not None and tiles[0] == 'u':
-        # one 16-row tile, number ``wave``: whole blocks
-        for b in range(4 // self.nb):
-          vals = ', '.join(f'{name}_0_0[{b * self.nb + j}]' for j in range(self.nb))
-          w(f'*reinterpret_cast<{self.lds_t}*>(ob + {c} * {self.out_lds_rows} + 16 * wave + '
-            f'{b * 4 * self.nb} + {self.nb} * g) = {self.lds_t}{{{vals}}};')
+    if self.post:
+      name = f'{name}p{len(self.post) - 1}'
+    if tiles is not None and tiles[0] == 'u':
+      # one 16-row tile, number ``wave``: whole blocks
+      for b in range(4 // self.nb):
+        vals = ', '.join(f'{name}_0_0[{b * self.nb + j}]' for j in range(self.nb))
+        w(f'*reinterpret_cast<{self.lds_t}*>(ob + {at} + 16 * wave + {b * 4 * self.nb} + '
+          f'{self.nb} * g) = {self.lds_t}{{{vals}}};')
+      return
+    held = None
+    if tiles is not None:
+      big = self.tiles(dr)[0]
+      held = [4 * t + x for t in tiles[1] for x in range(4)] + [4 * big + x for x in tiles[2]]
+    for st, base, n in dr.blocks():
+      if held is not None and st not in held:
         continue
-      held = None
-      if tiles is not None:
-        held = [4 * t + x for t in tiles[1] for x in range(4)] + [4 * big + x for x in tiles[2]]
-      for st, base, n in dr.blocks():
-        if held is not None and st not in held:
-          continue
-        refs = [self.acc_ref(name, 0, st + j) for j in range(n)]
-        if n == self.per:
-          w(f'*reinterpret_cast<{self.lds_t}*>(ob + {c} * {self.out_lds_rows} + {base} + '
-            f'{n} * g) = {self.lds_t}{{{", ".join(refs)}}};')
-        else:
-          for j in range(n):
-            w(f'ob[{c} * {self.out_lds_rows} + {base + j} + {n} * g] = {refs[j]};')
+      refs = [self.acc_ref(name, 0, st + j) for j in range(n)]
+      if n == self.per:
+        w(f'*reinterpret_cast<{self.lds_t}*>(ob + {at} + {base} + {n} * g) = '
+          f'{self.lds_t}{{{", ".join(refs)}}};')
+      else:
+        for j in range(n):
+          w(f'ob[{at} + {base + j} + {n} * g] = {refs[j]};')

@@ -182,3 +182,20 @@ def test_grouped_launch_takes_both_forms():
   except GenerationError as err:
     pytest.fail(str(err))
   assert grouped.block == (512, 1, 1)
+
+
+@pytest.mark.parametrize('tag', list(catalog.MATRIX_EDGES))
+def test_shares_of_a_ninth_quantity(tag):
+  e, program, pl = _form(f't_matrix_{tag}_auto')
+  k = staged._Staged(program, e.generator._context, 'x', pl)
+  if not k.prepare() or not k.shared_last:
+    return
+  for ph in k.phases:
+    # every block of the contraction belongs to one wavefront
+    full = [b for w in range(staged.SHARES) for b in range(w, ph.kr.full, staged.SHARES)]
+    assert sorted(full) == list(range(ph.kr.full))
+  # the other shares lie behind the results and inside the workgroup's LDS, a row run per element
+  assert k.share_base >= k.out.lds_base + tile.SET * k.out.lds_elem
+  end = k.share_base + (staged.SHARES - 1) * tile.SET * k.share_elem
+  assert k.share_elem >= k.out.lds_run and end <= k.lds_bytes // k.size
+  assert k.share_elem % k.per == 0 and k.share_base % k.per == 0
