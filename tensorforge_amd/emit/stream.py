@@ -492,6 +492,9 @@ class _Stream:
       self.dma_prologue()
     elif not self.loop:
       self.pipeline_prologue()
+      if self.early_weights():
+        w(f'{real} {", ".join(f"{v}_v" for slots in self.slots.values() for v, _ in slots)};')
+        self.load_weights('efirst')
     with w.block('for (size_t r = 0; r < rounds; ++r)'):
       w('const size_t e0 = efirst + r * estep;')
       w('const size_t e0n = e0 + estep;')
@@ -589,6 +592,58 @@ class _Stream:
         entries.append((v, self.offsets[ms]))
       self.slots[t_idx] = entries
 
+  def early_weights(self):
+    """The next group's weights are loaded before this group's results are stored. Loaded at the
+    top of the group they would wait for those stores: the memory counter is in order."""
+    return bool(self.slots) and not self.loop and not self.dma and \
+        all(t.W.arg.addressing == Addressing.STRIDED for t in self.pl.terms if t.kind == 'fused')
+
+  def weights(self, pointer, declare=''):
+    """Weights of the fused temporaries; their positions are recomputed from an opaque copy of
+    the lane's column each group, so they do not occupy registers across the loop."""
+    w = self.w
+    if self.slots:
+      w('int colr = col;')
+      w('asm volatile("" : "+v"(colr));')
+    for t_idx, slots in self.slots.items():
+      for v, _ in slots:
+        w(f'const int {v}_p = {self._select(self.positions[v]).replace("col ==", "colr ==")};')
+        w(f'const {self.real} {v}_x = ({self.real}){pointer(self.pl.terms[t_idx])}'
+          f'[{v}_p < 0 ? 0 : {v}_p];')
+        w(f'{declare}{v}_v = {v}_p >= 0 ? {v}_x : {self.lit(0)};')
+
+  def load_weights(self, ebase):
+    """Weights of the group at ``ebase``, in their registers when the block ends."""
+    w = self.w
+    with w.block(''):
+      w(f'const size_t ew = {ebase} + slot < numElements ? {ebase} + slot : 0;')
+      self.weights(lambda t: f'({t.W.arg.name} + ew * {t.W.arg.element_stride}ull + '
+                             f'{t.W.arg.name}_extraOffset)')
+    names = [f'{v}_v' for slots in self.slots.values() for v, _ in slots]
+    for n0 in range(0, len(names), 8):
+      ops = ', '.join(f'"+v"({n})' for n in names[n0:n0 + 8])
+      w(f'asm volatile("" : {ops});')
+
+  def touch_weights(self, ebase):
+    """One load per line of the next group's weights: they come into the L2 while the group's
+    products run."""
+    w = self.w
+    self.touched = []
+    with w.block(''):
+      w(f'const size_t ew = {ebase} + slot < numElements ? {ebase} + slot : 0;')
+      seen = set()
+      for t_idx, slots in self.slots.items():
+        a = self.pl.terms[t_idx].W.arg
+        ps = [p for v, _ in slots for p in self.positions[v] if p >= 0]
+        if a.name in seen or not ps:
+          continue
+        seen.add(a.name)
+        v = f'wt{len(self.touched)}'
+        self.touched.append(v)
+        at = f'{min(ps)} + col * {max(ps) - min(ps)} / {max(1, self.q - 1)}'
+        w(f'{v} = *reinterpret_cast<const unsigned*>({a.name} + ew * {a.element_stride}ull + '
+          f'{a.name}_extraOffset + {at});')
+
   def group_body(self):
     w = self.w
     pl = self.pl
@@ -604,17 +659,8 @@ class _Stream:
           f'{a.name}_extraOffset;')
       else:
         w(f'{ty}* __restrict__ g_{a.name} = {a.name}[eSafe] + {a.name}_extraOffset;')
-    # weights of the fused temporaries; their positions are recomputed from an opaque copy of
-    # the lane's column each group, so they do not occupy registers across the loop
-    if self.slots:
-      w('int colr = col;')
-      w('asm volatile("" : "+v"(colr));')
-    for t_idx, slots in self.slots.items():
-      t = pl.terms[t_idx]
-      for v, _ in slots:
-        w(f'const int {v}_p = {self._select(self.positions[v]).replace("col ==", "colr ==")};')
-        w(f'const {real} {v}_x = ({real})g_{t.W.arg.name}[{v}_p < 0 ? 0 : {v}_p];')
-        w(f'const {real} {v}_v = {v}_p >= 0 ? {v}_x : {self.lit(0)};')
+    if not self.early_weights():
+      self.weights(lambda t: f'g_{t.W.arg.name}', f'const {real} ')
     # destination column
     acc = 'acc'
     w(f'{real} {acc}[{rows}];')
@@ -652,8 +698,12 @@ class _Stream:
       self.declare_lane_pointers('e0', 'cur')
     if self.row_loads():
       self.row_offsets('e0', 'ro')
+    if self.early_weights():
+      w(f'unsigned {", ".join(f"wt{i}" for i in range(len(self.slots)))};')
     for bi, (b0, b1, only) in enumerate(self.blocks):
       w(f'// block [{b0}, {b1})' + (f' of term {only[0]}' if only else ''))
+      if bi == nb // 2 and self.early_weights():
+        self.touch_weights('e0n')
       # issue the loads of the block D ahead (this group's, or the next group's)
       tb = bi + D
       if tb < nb:
@@ -670,6 +720,10 @@ class _Stream:
       self.pipeline_write(nxt)
       self.pipeline_shift()
     self.pipeline_realign()
+    if self.early_weights():
+      ops = ', '.join(f'"v"({v})' for v in self.touched)
+      w(f'asm volatile("" :: {ops});')
+      self.load_weights('e0n')
     if pl.post:
       self.post_stages(acc)
       return
