@@ -25,10 +25,10 @@ Loads are issued without branches around them and waited for before the results 
 register written on two paths is copied where they meet, and the memory counter is in order, so
 either mistake turns the requests of the next set into waits (flux integral 428 us with both, 337
 without; derivative step 659 us with 21 spilled registers, 576 with none). Measured, vector form before / this form: C += A B, 56 x 56 by 56 x 9, 65,536 elements FP64
-208 / 138 us (5.7 TB/s); local flux integral, 131,072 elements 468 / 331 us (5.0 TB/s, which is what a
+208 / 138 us (5.7 TB/s); local flux integral, 131,072 elements 468 / 329 us (5.0 TB/s, which is what a
 plain copy of 56 of every 64 rows reaches); neighbour flux integral, 40,001 elements with a mask
-124 / 116 us; time-derivative step, 131,071 elements 618 / 549 us, three arrays, 50,000 elements
-293 / 252 us (both bound by the steps between the barriers of a set: two wavefronts per SIMD do not
+124 / 115 us; time-derivative step, 131,071 elements 618 / 543 us, three arrays, 50,000 elements
+293 / 249 us (both bound by the steps between the barriers of a set: two wavefronts per SIMD do not
 cover their LDS latencies).
 """
 from typing import Optional
@@ -744,7 +744,9 @@ class _Staged(_SetKernel, _Tile):
                 w(f'const {real} {copied} = {ops[j][ci]};')
                 ops[j][ci] = copied
           read(bi + 1)
-        w('__builtin_amdgcn_sched_barrier(0);')
+        # a fence behind the products of a term: with another before them the fragments are read
+        # only once the temporaries are formed (derivative step 556 us, now 543), without any the
+        # registers do not suffice (600)
         for j in range(n):
           self.step(s, f'{s.base + (st + j) * F}', cols, ops[j])
         w('__builtin_amdgcn_sched_barrier(0);')
