@@ -23,7 +23,7 @@ Per product ``out(:, j) = sum_k L(:, k) R(k, j)``:
 back to the plain emitter.
 """
 import math
-from dataclasses import asdict, dataclass, field
+from dataclasses import asdict, dataclass, field, replace
 from typing import Dict, List, Optional, Tuple
 
 from ..common.exceptions import GenerationError
@@ -858,6 +858,15 @@ def starved(emitted) -> bool:
   return (LDS_LIMIT // emitted.lds_bytes) * waves < 4
 
 
+def _equal_blocks(rows):
+  """Contraction block of the vector stream for FP32: blocks of equal length, at most 16 rows (a
+  lane's 64 bytes). Half the block boundaries of blocks of 8, whose registers FP32 does not need
+  (sparse volume chains, blocks of 8 / equal ones: 20 rows, 560,000 elements 342 / 323 us; 35 rows,
+  320,000 377 / 368; 42 rows, 266,666 391 / 367; 56 rows, 200,000 318 / 310; 64 rows, 175,000
+  399 / 391; 84 rows no difference)."""
+  return -(-rows // max(1, -(-rows // 16)))
+
+
 def emit(program, context, base_name, schedule=None) -> Emitted:
   from . import small, stream, tile
   schedule = schedule or Schedule(stream_matrix='auto')
@@ -870,7 +879,12 @@ def emit(program, context, base_name, schedule=None) -> Emitted:
     if pl is not None:
       sched = Schedule(**{**asdict(schedule), 'waves_per_block': schedule.stream_waves,
                           'k_block': schedule.stream_k_block})
-      emitted = stream.emit(program, context, base_name, sched, pl)
+      emitted = None
+      if schedule.stream_matrix == 'auto' and program.fp_type == FloatingPointType.FLOAT:
+        emitted = stream.emit(program, context, base_name,
+                              replace(sched, k_block=_equal_blocks(pl.khi - pl.klo)), pl)
+      if emitted is None or emitted.lds_bytes > LDS_LIMIT:
+        emitted = stream.emit(program, context, base_name, sched, pl)
       if emitted.lds_bytes <= LDS_LIMIT:
         if schedule.stream_matrix == 'auto':
           emitted.few = small.emit(program, context, base_name, sched, pl)
