@@ -46,7 +46,9 @@ def features(generator, candidate, batch, info):
   waves = sched.get('waves_per_block', knobs.get('waves_per_block', 1))
   per_block = max(1, em.elements_per_block)
   src = generator.get_kernel() or ''
-  sites = src.count('v_fmac_') + src.count('__builtin_fma') + src.count('fma(') + 1
+  # a builtin counts twice, in either type, as in the timed sweep
+  sites = src.count('v_fmac_') + src.count('__builtin_fma') + src.count('fma(') + \
+      src.count('fmaf(') + 1
   groups = batch / per_block / 256.0
   return [
     math.log2(batch), float(generator._context.fp_type == FloatingPointType.DOUBLE), nprod,
