@@ -441,7 +441,8 @@ class _Staged(_SetKernel, _Tile):
     if self.shared_last:
       self.lds_bytes = max(self.lds_bytes, end)
     cols = 1 if self.extra == 0 or self.shared_last or self.tiled_last else 2
-    acc = max((4 * self.tiles(s.dr)[0] + self.tiles(s.dr)[1]) for s in self.stages + self.post)
+    acc = max((4 * self.tiles(s.dr)[0] + self.tiles(s.dr)[1] * (1 if self.f64 else 5))
+              for s in self.stages + self.post)
     # the share's accumulators beside the own ones only over several phases
     acc = acc * (2 if self.shared_last and len(self.phases) > 1 else cols) + 4 * self.tiled_last
     # registers (32-bit): accumulators, operands on the way, streamed rows, weights
@@ -650,6 +651,8 @@ class _Staged(_SetKernel, _Tile):
     if ph.kr.tail:
       with w.block(f'if (wave == {ph.kr.full % SHARES})'):
         block(ph.kr.full * self.nb, ph.kr.full * 4 * self.nb, ph.kr.tail)
+    if pi == len(self.phases) - 1:
+      self.finish('acx', self.stages[-1].dr, [0])
 
   def compute_columns(self, pi, cols):
     w = self.w
@@ -750,6 +753,10 @@ class _Staged(_SetKernel, _Tile):
         for j in range(n):
           self.step(s, f'{s.base + (st + j) * F}', cols, ops[j])
         w('__builtin_amdgcn_sched_barrier(0);')
+    if last:
+      for name, _, tiles in cols:
+        self.finish(name, self.stages[-1].dr, [0],
+                    None if tiles is None else ((), tiles[2] if tiles[0] == 'r' else ()))
     if last and self.post:
       prev_stage = self.stages[-1]
       for i, s in enumerate(self.post):
@@ -760,6 +767,8 @@ class _Staged(_SetKernel, _Tile):
         for j in range(s.kr.steps):
           self.step(s, f'{s.base + j * self.fragment(s.dr)}',
                     [(f'{name}p{i}', c, t) for name, c, t in cols], [o[j][0] for o in per_col])
+        for name, _, _ in cols:
+          self.finish(f'{name}p{i}', s.dr, [0])
         prev_stage = s
 
   def step(self, s, off, cols, ops):
@@ -780,7 +789,7 @@ class _Staged(_SetKernel, _Tile):
       w(f'const {self.real} {a} = ks[{off} + {64 * big + 16 * i}];')
       for name, op in whole + [(nm, op) for nm, tiles, op in rest
                                if tiles[0] == 'r' and i in tiles[2]]:
-        w(f'{name}_0s{i} = __builtin_amdgcn_mfma_f64_4x4x4f64({a}, {op}, {name}_0s{i}, 0, 0, 0);')
+        self.mfma_small(f'{name}_0', i, a, op)
     for name, tiles, op in rest:
       if tiles[0] == 'u':
         a = self.fresh('xa')

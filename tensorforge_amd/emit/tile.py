@@ -32,7 +32,7 @@ What bounds it: FP64 matrix instructions and FP64 FMAs share one unit (measured 
 at its two wavefronts per SIMD and pays for the address of every lane's own cache line. FP32 matrix
 instructions run at 125-150 TF beside the vector unit. Measured on MI355X, vector form before / this
 form: order-6 volume chain with dense K_d, 65,536 elements FP64 335 / 206 us (57 TF), 100,003
-elements FP32 409 / 179 us (99 TF); order 7, 30,000 elements FP64 432 / 235 us. Matrix instructions
+elements FP32 409 / 177 us (100 TF); order 7, 30,000 elements FP64 432 / 235 us. Matrix instructions
 are issued 62 % of the cycles there, the FP64 FMAs of the temporaries take another 5 %; fragments
 read further ahead, the next term's temporaries formed among the matrix instructions, or rows
 shared through LDS (a barrier per block) did not change or lost time.
@@ -209,11 +209,14 @@ class _Tile:
   def tiles(self, dr: Rows):
     """(16-row tiles, 4-row tiles) of a destination row range. The FP64 matrix core runs a 4-row
     tile of four column blocks (v_mfma_f64_4x4x4_4b, 16 cycles) at the 16-row tile's rate (64
-    cycles) with the same B and D registers, so FP64 rows are padded to 4; FP32 has no such form:
-    16."""
-    if self.f64:
-      return dr.steps // 4, dr.steps % 4
-    return _ceil(dr.steps, 4), 0
+    cycles) with the same B and D registers. The FP32 one (v_mfma_f32_4x4x1_16b, 8 cycles against
+    32) multiplies each lane group's contraction row into sums of its own: four registers, added
+    over the lane groups when the contraction ends (:meth:`finish`). Three of them take more
+    registers than they save (dense volume chains FP32, last rows in 16-row / 4-row tiles: 10 rows,
+    3 tiles 50 / 54 us; 20 rows, 1 tile 123 / 110; 35 rows, 1 tile 330 / 311; 56 rows, 2 tiles 180 /
+    178; 84 rows, 1 tile 419 / 389)."""
+    big, small = dr.steps // 4, dr.steps % 4
+    return (big, small) if self.f64 or small < 3 else (big + 1, 0)
 
   def fragment(self, dr):
     """LDS entries of one contraction step's A operand."""
@@ -222,7 +225,7 @@ class _Tile:
 
   def acc_registers(self, dr):
     big, small = self.tiles(dr)
-    return (4 * big + small) * (self.size // 4) * len(self.halves[0])
+    return (4 * big + small * (1 if self.f64 else 5)) * (self.size // 4) * len(self.halves[0])
 
   def weights(self, t, half):
     """[(column, [(m, position)])] of term t's stored weights in the half's columns."""
@@ -407,17 +410,19 @@ class _Tile:
     # every value on a line of its own: a conditional expression of such terms becomes a branch,
     # and a branch between two entries keeps their loads apart
     lines = [f'const int st = e / {F};', f'const int f = e - st * {F};']
+    # 16-row tiles, then 4-row tiles
     if self.f64:
-      # 16-row tiles, then 4-row tiles
-      lines += ['const int j1 = f / 64 * 4 + f % 16 / 4;', 'const int kg1 = f % 64 / 16;',
-                f'const int j2 = {4 * big} + (f - {64 * big}) / 16;',
-                f'const int kg2 = (f - {64 * big}) % 16 / 4;',
-                f'const int j = f < {64 * big} ? j1 : j2;',
-                f'const int kg = f < {64 * big} ? kg1 : kg2;', 'const int g = f % 4;']
+      lines += ['const int j1 = f / 64 * 4 + f % 16 / 4;', 'const int g1 = f % 4;',
+                f'const int j2 = {4 * big} + (f - {64 * big}) / 16;', 'const int g2 = g1;']
     else:
-      lines += ['const int j = f / 64 * 4 + f % 4;', 'const int g = f % 16 / 4;',
-                'const int kg = f % 64 / 16;']
-    # FP32 tiles have four registers; those past the last block's steps hold no row
+      # (a 4-row tile's rows follow each other: entry x of the last block's 4 n rows)
+      n = max(1, small)
+      lines += ['const int j1 = f / 64 * 4 + f % 4;', 'const int g1 = f % 16 / 4;',
+                f'const int x = (f - {64 * big}) / 16 * 4 + f % 4;',
+                f'const int j2 = {4 * big} + x % {n};', f'const int g2 = x / {n};']
+    lines += ['const int kg1 = f % 64 / 16;', f'const int kg2 = (f - {64 * big}) % 16 / 4;',
+              f'const int j = f < {64 * big} ? j1 : j2;', f'const int g = f < {64 * big} ? g1 : g2;',
+              f'const int kg = f < {64 * big} ? kg1 : kg2;']
     lines += [f'const int row = {s.dr.row_sum("j", "g")};',
               f'const int k = {s.kr.row_sum("st", "kg")} + {s.k0};',
               f'const bool in = (j < {s.dr.steps}) & (row < {nrows}) & (k >= {s.krange[0]}) & '
@@ -554,6 +559,7 @@ class _Tile:
         self.declare_acc('acc', stages[0].dr, half)
       for pi in range(len(phases)):
         self.phase(pi, half, plan, 'acc')
+      self.finish('acc', stages[-1].dr, half)
       prev, prev_stage = 'acc', stages[-1]
       for si, s in enumerate(post[:-1]):
         name = f'acp{si}'
@@ -561,6 +567,7 @@ class _Tile:
         ops = self.post_operands(s, prev, prev_stage, half)
         for j in range(s.kr.steps):
           self.mfma(name, s, f'{s.base + j * self.fragment(s.dr)}', ops[j])
+        self.finish(name, s.dr, half)
         prev, prev_stage = name, s
       if not post:
         with w.block('if (act)'):
@@ -573,6 +580,7 @@ class _Tile:
           w('__builtin_amdgcn_sched_barrier(0);')
           for j in range(last.kr.steps):
             self.mfma('out', last, f'{last.base + j * self.fragment(last.dr)}', ops[j], chunk)
+          self.finish('out', last.dr, half, chunk)
           with w.block('if (act)'):
             self.dest_rows('out', last.dr, half, last.rows, 'store', 1.0, chunk)
           w('__builtin_amdgcn_sched_barrier(0);')
@@ -589,11 +597,6 @@ class _Tile:
   # ------------------------------------------------------------------ accumulators
   def acc_ref(self, name, c, j):
     """Result register j of quantity c."""
-    if self.f64:
-      return self._acc64(name, c, j)
-    return f'{name}_{c}_{j // 4}[{j % 4}]'
-
-  def _acc64(self, name, c, j):
     big = self.acc_big[name]
     return f'{name}_{c}_{j // 4}[{j % 4}]' if j < 4 * big else f'{name}_{c}s{j - 4 * big}'
 
@@ -617,6 +620,8 @@ class _Tile:
         w(f'{self.acc_t} {name}_{c}_{t} = {{{zero}, {zero}, {zero}, {zero}}};')
       for s in small:
         w(f'{self.real} {name}_{c}s{s} = {zero};')
+        if not self.f64:
+          w(f'{self.acc_t} {name}_{c}q{s} = {{{zero}, {zero}, {zero}, {zero}}};')
 
   def open_chunk(self, name, s, chunk, half):
     self.declare_acc(name, s.dr, half, chunk)
@@ -692,7 +697,36 @@ class _Tile:
       a = self.fresh('xa')
       w(f'const {self.real} {a} = ks[{step_off} + {64 * self.tiles(s.dr)[0] + 16 * i}];')
       for c, b in operands.items():
-        w(f'{name}_{c}s{i} = __builtin_amdgcn_mfma_f64_4x4x4f64({a}, {b}, {name}_{c}s{i}, 0, 0, 0);')
+        self.mfma_small(f'{name}_{c}', i, a, b)
+
+  def mfma_small(self, name, i, a, b):
+    if self.f64:
+      self.w(f'{name}s{i} = __builtin_amdgcn_mfma_f64_4x4x4f64({a}, {b}, {name}s{i}, 0, 0, 0);')
+    else:
+      self.w(f'{name}q{i} = __builtin_amdgcn_mfma_f32_4x4x1f32({a}, {b}, {name}q{i}, 0, 0, 0);')
+
+  def finish(self, name, dr, half, chunk=None):
+    """The lane groups' sums of the FP32 4-row tiles, added up and dealt out: entry x of the 4 n rows
+    of the last block ends in group x / n. Two exchanges, of half the wavefront and of neighbouring
+    groups, each halving the number of registers."""
+    w = self.w
+    small = (chunk or self.all_tiles(dr))[1]
+    n = len(small)
+    if self.f64 or not n:
+      return
+    for c in half:
+      x = [f'{name}_{c}q{t}[{i}]' for t in small for i in range(4)]
+      for swap, count in (('32', 2 * n), ('16', n)):
+        y = []
+        for r in range(count):
+          p, v = self.fresh('xe'), self.fresh('xf')
+          w(f'const auto {p} = __builtin_amdgcn_permlane{swap}_swap(__float_as_uint({x[r]}), '
+            f'__float_as_uint({x[r + count]}), false, false);')
+          w(f'const float {v} = __uint_as_float({p}[0]) + __uint_as_float({p}[1]);')
+          y.append(v)
+        x = y
+      for j in range(n):
+        w(f'{name}_{c}s{j} += {x[j]};')
 
   def stage_weights(self, ph, half):
     """The wavefront's weights of the phase's terms into its LDS region, [position][element]."""
@@ -894,7 +928,8 @@ def set_times(program, pl):
 
   def cycles(k, rows):
     steps = Rows(rows, nb).steps
-    per = (64 * (steps // 4) + 16 * (steps % 4)) if f64 else 32 * _ceil(steps, 4)
+    per = 64 * (steps // 4) + 16 * (steps % 4) if f64 else \
+        32 * (steps // 4) + (8 * (steps % 4) if steps % 4 < 3 else 32)
     return Rows(k, nb).steps * per
   rows = pl.rows[1] - pl.rows[0]
   total = sum(cycles(t.product.k_ranges[0][1] - t.product.k_ranges[0][0], rows) for t in pl.terms)

@@ -199,3 +199,23 @@ def test_shares_of_a_ninth_quantity(tag):
   end = k.share_base + (staged.SHARES - 1) * tile.SET * k.share_elem
   assert k.share_elem >= k.out.lds_run and end <= k.lds_bytes // k.size
   assert k.share_elem % k.per == 0 and k.share_base % k.per == 0
+
+
+@pytest.mark.parametrize('n', [1, 2])
+def test_lane_group_sums_are_dealt_out(n):
+  """The exchanges of ``finish`` on four lane groups, ``[register][group]``."""
+  import numpy as np
+  part = np.random.default_rng(n).integers(-9, 9, (4 * n, 4))
+
+  def swap(a, b, rows):
+    """Odd ``rows``-groups of a against even ones of b (halves: 2 groups, neighbours: 1)."""
+    a2, b2 = a.copy(), b.copy()
+    for g in range(0, 4, 2 * rows):
+      a2[g + rows:g + 2 * rows], b2[g:g + rows] = b[g:g + rows], a[g + rows:g + 2 * rows]
+    return a2, b2
+  x = list(part)
+  for rows, count in ((2, 2 * n), (1, n)):
+    x = [sum(swap(x[r], x[r + count], rows)) for r in range(count)]
+  for g in range(4):
+    for j in range(n):
+      assert x[j][g] == part[n * g + j].sum()
