@@ -267,7 +267,6 @@ class _Tile:
     off = 0
     for s in stages + post:
       s.base = off
-      # FP32 result tiles always have four registers: a product of the chain steps over all of them
       off += s.kr.steps * self.fragment(s.dr)
     phases = []
     if self.fused and not split_terms:
