@@ -36,6 +36,25 @@ void launcher_kernel_368dd01f68(float* m0, unsigned m0_extraOffset, const float*
 #elif defined(TF_CATALOG_GEMM_F64_MFMA_FP64) || defined(TF_CATALOG_GEMM_F64_PLAIN) || defined(TF_CATALOG_GEMM_F64_TUNED) || defined(TF_CATALOG_OPT_GEMM_F64_K4) || defined(TF_CATALOG_OPT_GEMM_F64_LA0) || defined(TF_CATALOG_OPT_GEMM_F64_MFMA64W4K8REGS) || defined(TF_CATALOG_OPT_GEMM_F64_MFMA64W8K8ACC) || defined(TF_CATALOG_OPT_GEMM_F64_MFMA64W8K8END) || defined(TF_CATALOG_OPT_GEMM_F64_PAIR) || defined(TF_CATALOG_OPT_GEMM_F64_PF2) || defined(TF_CATALOG_OPT_GEMM_F64_W4)
 void launcher_kernel_368dd01f68(double* m0, unsigned m0_extraOffset, const double* m1, const double* m2, unsigned m2_extraOffset, size_t numElements, unsigned* flags, void* streamPtr);
 #endif
+/* inplace_chain_20x70 */
+void launcher_kernel_50ca05ee0c(double* m0, unsigned m0_extraOffset, const double* m1, unsigned m1_extraOffset, const double* m2, const double* m3, size_t numElements, unsigned* flags, void* streamPtr);
+/* inplace_gemm_41_sparse */
+void launcher_kernel_2e103479a9(double* m0, unsigned m0_extraOffset, const double* m1, size_t numElements, unsigned* flags, void* streamPtr);
+/* inplace_gemm_56 */
+void launcher_kernel_79587ab2d2(double* m0, unsigned m0_extraOffset, const double* m1, size_t numElements, unsigned* flags, void* streamPtr);
+/* inplace_gemm_70_q30 */
+void launcher_kernel_60bfedee1e(double* m0, unsigned m0_extraOffset, const double* m1, size_t numElements, unsigned* flags, void* streamPtr);
+#if defined(TF_CATALOG_INPLACE_GEMM_84_Q13)
+void launcher_kernel_ef20024dca(double* m0, unsigned m0_extraOffset, const double* m1, size_t numElements, unsigned* flags, void* streamPtr);
+#elif defined(TF_CATALOG_INPLACE_GEMM_84_Q13_F32)
+void launcher_kernel_ef20024dca(float* m0, unsigned m0_extraOffset, const float* m1, size_t numElements, unsigned* flags, void* streamPtr);
+#endif
+/* inplace_volume_20 */
+void launcher_kernel_b042afe2ce(double* m0, unsigned m0_extraOffset, const double* m1, unsigned m1_extraOffset, const double* m2, size_t numElements, unsigned* flags, void* streamPtr);
+/* inplace_volume_70_f32 */
+void launcher_kernel_00f28504d5(float* m0, unsigned m0_extraOffset, const float* m1, unsigned m1_extraOffset, const float* m2, size_t numElements, unsigned* flags, void* streamPtr);
+/* inplace_volume_84 */
+void launcher_kernel_db3b423e76(double* m0, unsigned m0_extraOffset, const double* m1, unsigned m1_extraOffset, const double* m2, size_t numElements, unsigned* flags, void* streamPtr);
 /* pw_clamp_scale_f64 */
 void launcher_kernel_b29a95e19f(double* m0, unsigned m0_extraOffset, double m1, size_t numElements, unsigned* flags, void* streamPtr);
 /* pw_plastic_f64 */

@@ -616,6 +616,48 @@ for _tag, _kw in FEW_EDGES.items():
 _auto_variants()
 
 
+def _in_place_entry(kind, m, q=9, fp=F64, sparse=False, mid=0):
+  """Chains that read the tensor they write: ``gemm`` D = K D, ``volume`` D = K (D S), ``chain``
+  D += V (U (D S)) with ``mid`` rows between."""
+  pair, ident = [[0, -1], [-1, 1]], [[0, 1], [0, 1]]
+  D = _t([m, q], Addressing.STRIDED, alias='D')
+  mask = ListSPP([(r, c) for c in range(m) for r in range(m) if (2 * r + 3 * c) % 5 < 2],
+                 (m, m)) if sparse else None
+  K = _t([m, mid or m], Addressing.NONE, spp=mask, alias='K')
+  tensors = {'D': D, 'K': K}
+  descrs, right = [], _sub(D)
+  if kind != 'gemm':
+    S = _t([q, q], Addressing.STRIDED, alias='S')
+    tensors['S'] = S
+    T = generate_tmp_tensor([right, _sub(S)], pair)
+    descrs.append(MultilinearDescr(_sub(T), [right, _sub(S)], pair, ident))
+    right = _sub(T)
+  if kind == 'chain':
+    U = _t([mid, m], Addressing.NONE, alias='U')
+    tensors['U'] = U
+    T = generate_tmp_tensor([_sub(U), right], pair)
+    descrs.append(MultilinearDescr(_sub(T), [_sub(U), right], pair, ident))
+    right = _sub(T)
+  descrs.append(MultilinearDescr(_sub(D), [_sub(K), right], pair, ident, add=kind == 'chain'))
+  return Entry('', descrs, fp, tensors)
+
+
+# at the sizes where the forms divide a destination into row bands, and below them
+IN_PLACE = {
+  'gemm_56': dict(kind='gemm', m=56),
+  'gemm_41_sparse': dict(kind='gemm', m=41, sparse=True),
+  'gemm_84_q13': dict(kind='gemm', m=84, q=13),
+  'gemm_84_q13_f32': dict(kind='gemm', m=84, q=13, fp=F32),
+  'gemm_70_q30': dict(kind='gemm', m=70, q=30),
+  'volume_20': dict(kind='volume', m=20),
+  'volume_70_f32': dict(kind='volume', m=70, fp=F32),
+  'volume_84': dict(kind='volume', m=84),
+  'chain_20x70': dict(kind='chain', m=20, mid=70),
+}
+for _tag, _kw in IN_PLACE.items():
+  register(f'inplace_{_tag}')(lambda kw=_kw: _in_place_entry(**kw))
+
+
 # ---- pointwise kernels (ElementwiseDescr) ----
 for _fp, _fpn in ((F64, 'f64'), (F32, 'f32')):
   register(f'pw_update_{_fpn}')(lambda fp=_fp: _wl_entry(W.pointwise_update(fp), 'auto'))

@@ -1606,12 +1606,27 @@ class _Stream:
       w(f'{acc} = {self.fp.fma()}({b}, {r}, {acc});')
 
 
+def in_place(pl):
+  """The chain reads rows that it writes: its destination is the streamed operand, a weight, or a
+  right operand whose contraction rows are among the destination's."""
+  rows = pl.post[-1].rows if pl.post else pl.rows
+  for t in pl.terms:
+    if t.kind == 'fused':
+      if (t.L or pl.L).arg is pl.dest or t.W.arg is pl.dest:
+        return True
+    elif t.B.arg is pl.dest and max(rows[0], pl.klo) < min(rows[1], pl.khi):
+      return True
+  return False
+
+
 def _row_passes(pl, schedule):
   """Row ranges of the passes: one pass unless the destination has more rows than
-  ``stream_pass_rows`` and its shared operands are dense (the runtime block loop)."""
+  ``stream_pass_rows`` and its shared operands are dense (the runtime block loop). A chain in place
+  has one pass: a second one would read what the first one wrote."""
   rows = pl.rows[1] - pl.rows[0]
   limit = schedule.stream_pass_rows
-  if limit <= 0 or rows <= limit or any(t.U.is_sparse() for t in pl.terms):
+  if limit <= 0 or rows <= limit or any(t.U.is_sparse() for t in pl.terms) or \
+      in_place(pl):
     return [pl.rows]
   n = (rows + limit - 1) // limit
   step = (rows + n - 1) // n

@@ -43,6 +43,7 @@ from typing import List, Optional
 from ..common.basic_types import Addressing, FloatingPointType
 from . import ir
 from .launcher import Emitted, Writer, fill_shared, kernel_params, persistent_grid
+from .stream import in_place
 from .traffic import element_traffic
 
 WAVE = 64
@@ -296,7 +297,8 @@ class _Tile:
     as the last resort the terms one after the other, reading the streamed rows once per term."""
     pl = self.pl
     n = pl.rows[1] - pl.rows[0]
-    max_bands = 1 if pl.post else 4
+    # (a second band of a product in place would read what the first one wrote)
+    max_bands = 1 if pl.post or in_place(pl) else 4
     for bands in range(1, max_bands + 1):
       step = _ceil(_ceil(n, bands), 4) * 4
       windows = [(r, min(r + step, pl.rows[1])) for r in range(pl.rows[0], pl.rows[1], step)]
