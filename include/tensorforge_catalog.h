@@ -55,6 +55,8 @@ void launcher_kernel_b042afe2ce(double* m0, unsigned m0_extraOffset, const doubl
 void launcher_kernel_00f28504d5(float* m0, unsigned m0_extraOffset, const float* m1, unsigned m1_extraOffset, const float* m2, size_t numElements, unsigned* flags, void* streamPtr);
 /* inplace_volume_84 */
 void launcher_kernel_db3b423e76(double* m0, unsigned m0_extraOffset, const double* m1, unsigned m1_extraOffset, const double* m2, size_t numElements, unsigned* flags, void* streamPtr);
+/* opt_t_matrix_chain_20x70x20_vector, t_matrix_chain_20x70x20_auto, t_matrix_chain_20x70x20_plain */
+void launcher_kernel_4507257447(const double* m0, unsigned m0_extraOffset, const double* m1, unsigned m1_extraOffset, const double* m2, double* m3, unsigned m3_extraOffset, const double* m4, size_t numElements, unsigned* flags, void* streamPtr);
 /* pw_clamp_scale_f64 */
 void launcher_kernel_b29a95e19f(double* m0, unsigned m0_extraOffset, double m1, size_t numElements, unsigned* flags, void* streamPtr);
 /* pw_plastic_f64 */

@@ -595,6 +595,8 @@ MATRIX_EDGES = {
   'chain_13x6x29_q4': dict(kind='chain', m=13, mid=6, k=29, q=4, beta=1.0),
   'chain_37x18x50_f32': dict(kind='chain', m=37, mid=18, k=50, q=9, fp=F32, beta=1.0,
                              dense_star=True),
+  # more rows between the shared operands than the vector stream takes in one band of a product
+  'chain_20x70x20': dict(kind='chain', m=20, mid=70, k=20, q=9, beta=1.0),
 }
 for _tag, _kw in MATRIX_EDGES.items():
   register(f't_matrix_{_tag}_plain')(lambda kw=_kw: _matrix_entry(**kw))
@@ -744,6 +746,8 @@ for _tag, _kw in STREAM_OPTIONS.items():
     register(f'opt_gemm_f64_{_tag}')(lambda kw=_kw: _option_entry(W.gemm(F64), kw))
 register('opt_ader_dense_f64_unrolled')(
   lambda: _option_entry(W.ader_volume(F64, sparse_k=False), dict(stream_loop='never')))
+register('opt_t_matrix_chain_20x70x20_vector')(
+  lambda: _option_entry(_matrix_entry(**MATRIX_EDGES['chain_20x70x20']), {}))
 
 
 @register('t_pw_big')

@@ -1622,11 +1622,12 @@ def in_place(pl):
 def _row_passes(pl, schedule):
   """Row ranges of the passes: one pass unless the destination has more rows than
   ``stream_pass_rows`` and its shared operands are dense (the runtime block loop). A chain in place
-  has one pass: a second one would read what the first one wrote."""
+  has one pass (a second one would read what the first one wrote), and so has a chain with register
+  stages (they need every row of the streamed product)."""
   rows = pl.rows[1] - pl.rows[0]
   limit = schedule.stream_pass_rows
   if limit <= 0 or rows <= limit or any(t.U.is_sparse() for t in pl.terms) or \
-      in_place(pl):
+      pl.post or in_place(pl):
     return [pl.rows]
   n = (rows + limit - 1) // limit
   step = (rows + n - 1) // n
