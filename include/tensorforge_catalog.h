@@ -23,6 +23,8 @@ void launcher_kernel_b053681baa(const double* m0, unsigned m0_extraOffset, const
 void launcher_kernel_7d2f2effa5(const double* m0, unsigned m0_extraOffset, const double* m1, unsigned m1_extraOffset, double* m2, unsigned m2_extraOffset, const double* m3, const double* m4, unsigned m4_extraOffset, const double* m5, const double* m6, unsigned m6_extraOffset, const double* m7, size_t numElements, unsigned* flags, void* streamPtr);
 /* deriv_na_f64_plain, deriv_na_f64_tuned */
 void launcher_kernel_e957b6379b(const double* m0, unsigned m0_extraOffset, const double* m1, unsigned m1_extraOffset, double* m2, unsigned m2_extraOffset, const double* m3, const double* m4, unsigned m4_extraOffset, const double* m5, unsigned m5_extraOffset, const double* m6, const double* m7, unsigned m7_extraOffset, const double* m8, unsigned m8_extraOffset, const double* m9, size_t numElements, unsigned* flags, void* streamPtr);
+/* few_empty_term */
+void launcher_kernel_cca5f863e5(const double* m0, unsigned m0_extraOffset, const double* m1, unsigned m1_extraOffset, double* m2, unsigned m2_extraOffset, const double* m3, const double* m4, unsigned m4_extraOffset, const double* m5, const double* m6, unsigned m6_extraOffset, const double* m7, const double* m8, unsigned m8_extraOffset, const double* m9, size_t numElements, unsigned* flags, void* streamPtr);
 /* flux_local_mod_f64_plain, flux_local_mod_f64_tuned */
 void launcher_kernel_28ade16a80(const double* m0, unsigned m0_extraOffset, const double* m1, unsigned m1_extraOffset, const double* m2, double* m3, unsigned m3_extraOffset, const double* m4, size_t numElements, unsigned* flags, void* streamPtr);
 /* flux_local_orig_f64_plain, flux_local_orig_f64_tuned */

@@ -660,6 +660,24 @@ for _tag, _kw in IN_PLACE.items():
   register(f'inplace_{_tag}')(lambda kw=_kw: _in_place_entry(**kw))
 
 
+@register('few_empty_term')
+def _few_empty_term_entry():
+  """D = sum_t K_t (Q S_t) whose second and third K_t store nothing (their buffers may be empty)."""
+  pair, ident = [[0, -1], [-1, 1]], [[0, 1], [0, 1]]
+  Q = _t([12, 9], Addressing.STRIDED, alias='Q')
+  D = _t([12, 9], Addressing.STRIDED, alias='D')
+  tensors, descrs = {'Q': Q, 'D': D}, []
+  for i in range(4):
+    stored = [(r, c) for c in range(12) for r in range(12) if (r + c + i) % 3 == 0 and i in (0, 3)]
+    S = _t([9, 9], Addressing.STRIDED, alias=f'S{i}')
+    K = _t([12, 12], Addressing.NONE, spp=ListSPP(stored, (12, 12)), alias=f'K{i}')
+    T = generate_tmp_tensor([_sub(Q), _sub(S)], pair)
+    descrs.append(MultilinearDescr(_sub(T), [_sub(Q), _sub(S)], pair, ident))
+    descrs.append(MultilinearDescr(_sub(D), [_sub(K), _sub(T)], pair, ident, add=i > 0))
+    tensors.update({f'S{i}': S, f'K{i}': K})
+  return Entry('', descrs, F64, tensors)
+
+
 # ---- pointwise kernels (ElementwiseDescr) ----
 for _fp, _fpn in ((F64, 'f64'), (F32, 'f32')):
   register(f'pw_update_{_fpn}')(lambda fp=_fp: _wl_entry(W.pointwise_update(fp), 'auto'))

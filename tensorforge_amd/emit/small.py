@@ -135,10 +135,13 @@ class _Small(_SetKernel):
     # per term (first position, entries, offset)
     self.raw, n = [], 0
     for ti in range(len(pl.terms)):
-      ps = [s[2][2] for p in self.parts for s in p.seq if s[1] == ti] or [0]
-      self.raw.append((min(ps), max(ps) + 1 - min(ps), n))
-      n += max(ps) + 1 - min(ps)
+      ps = [s[2][2] for p in self.parts for s in p.seq if s[1] == ti]
+      first, cnt = (min(ps), max(ps) + 1 - min(ps)) if ps else (0, 0)
+      self.raw.append((first, cnt, n))
+      n += cnt
     self.raw_total, self.total = n, chunk * CHUNK
+    if n == 0:
+      return False
     words = self.tbase + max(n, len(pl.terms) * rows * WAVE if self.fused else 0)
     if _ceil(self.total, THREADS) > 64:
       return False
