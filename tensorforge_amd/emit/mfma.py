@@ -112,6 +112,10 @@ def unsupported_reason(program, pl, mode='fp32', sched=None):
     return 'a per-element operand is not strided'
   if program.epilogue is not None:
     return 'pointwise statements fused into the chain'
+  from .tuned import read_after_write
+  reason = read_after_write(program)
+  if reason is not None:
+    return reason
   waves, kb = _shape(pl, mode, sched)
   if waves not in (4, 8) or kb not in ((8, 16) if mode == 'fp64' else (KB,)):
     return f'{waves} wavefronts with {kb}-row blocks'

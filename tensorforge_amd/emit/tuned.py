@@ -209,7 +209,12 @@ def unsupported_reason(program: ir.ChainProgram, context, schedule=None):
       return 'temporary with offset columns'
   if ncols is None:
     return 'no products'
-  # a global destination read back as an operand later in the chain
+  return read_after_write(program)
+
+
+def read_after_write(program):
+  """A global destination read back as an operand later in the chain, or None: every form but the
+  plain one reads the operands of all products before it writes."""
   written = set()
   for p in program.products:
     for f in p.factors:

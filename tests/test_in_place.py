@@ -28,6 +28,32 @@ def test_bands_where_nothing_is_read_back():
   assert e.generator.get_emitted().schedule['row_passes'] == 2
 
 
+def test_matrix_core_forms_by_name_refuse_a_second_product_in_place():
+  """Its right operand is what the first product wrote."""
+  from tensorforge_amd.common.aux import generate_tmp_tensor
+  from tensorforge_amd.common.basic_types import Addressing, FloatingPointType
+  from tensorforge_amd.common.context import Context
+  from tensorforge_amd.common.exceptions import GenerationError
+  from tensorforge_amd.common.matrix.tensor import SubTensor, Tensor
+  from tensorforge_amd.generators.descriptions import MultilinearDescr
+  from tensorforge_amd.generators.generator import Generator
+  pair, ident = [[0, -1], [-1, 1]], [[0, 1], [0, 1]]
+  D = Tensor([20, 9], Addressing.STRIDED, alias='D')
+  descrs = []
+  for i in range(2):
+    S = Tensor([9, 9], Addressing.STRIDED, alias=f'S{i}')
+    K = Tensor([20, 20], Addressing.NONE, alias=f'K{i}')
+    T = generate_tmp_tensor([SubTensor(D), SubTensor(S)], pair)
+    descrs += [MultilinearDescr(SubTensor(T), [SubTensor(D), SubTensor(S)], pair, ident),
+               MultilinearDescr(SubTensor(D), [SubTensor(K), SubTensor(T)], pair, ident, add=i > 0)]
+  for emitter in ('mfma_fp64', 'mfma_fp32', 'mfma_bf16x3'):
+    g = Generator(descrs, Context('gfx950', 'hip', FloatingPointType.DOUBLE), emitter=emitter)
+    with pytest.raises(GenerationError, match='read after the chain writes it'):
+      g.generate()
+    Generator(descrs[:2], Context('gfx950', 'hip', FloatingPointType.DOUBLE),
+              emitter=emitter).generate()
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize('tag', list(catalog.IN_PLACE))
 def test_against_the_oracle(tag, device):
