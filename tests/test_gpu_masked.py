@@ -1,0 +1,50 @@
+"""Masked launches and extra offsets through the matrix-core and vector forms of both types.
+
+60,001 elements (several rounds of a workgroup, a partial last set), every per-element operand behind
+an odd number of unused entries, masks that skip single elements, whole sets of 16 and everything;
+every element is compared with the plain launcher of the same chain. Normwise per element 1e-12
+FP64, 1e-5 FP32.
+"""
+import numpy as np
+import pytest
+
+from tensorforge_amd import catalog
+
+from harness import TOL, gpu_run, key_of, make_inputs, normwise_error, outputs_of
+
+pytestmark = pytest.mark.gpu
+
+N = 60001
+MASKS = {
+  'single': np.arange(N) % 5 != 3,
+  'runs': np.arange(N) // 37 % 3 == 1,
+  'few': np.arange(N) % 1013 == 7,
+  'none': np.zeros(N, bool),
+}
+ENTRIES = ['ader_f32_tuned', 'ader_dense_f64_tuned', 'ader_dense_f32_tuned', 'ader7_f64_tuned',
+           'gemm_f64_tuned', 'gemm_f32_tuned', 'flux_local_mod_f64_tuned',
+           'flux_neigh_mod_f64_tuned', 'deriv_f64_tuned', 'deriv_na_f64_tuned']
+ENTRIES += [f't_matrix_{t}_auto' for t in catalog.MATRIX_EDGES]
+
+
+@pytest.mark.parametrize('name', ENTRIES)
+def test_masked_with_offsets(name, device):
+  et, kt = catalog.load(name)
+  ep, kp = catalog.load(name.rsplit('_', 1)[0] + '_plain')
+  keys = [key_of(t) for t in ep.generator._global_tensors if t.addressing.name == 'STRIDED']
+  offsets = {k: 3 + 2 * i for i, k in enumerate(keys)}
+  host = make_inputs(ep, N, seed=29, offsets=offsets)
+  for tag, mask in MASKS.items():
+    flags = mask.astype(np.uint32)
+    print(f'{name}: mask {tag}', flush=True)
+    a = gpu_run(kp, ep, host, N, device, offsets=offsets, flags=flags)
+    b = gpu_run(kt, et, host, N, device, offsets=offsets, flags=flags)
+    for t in ep.generator._global_tensors:
+      key = key_of(t)
+      if key not in outputs_of(ep):
+        continue
+      off, vol = offsets.get(key, 0), t.get_real_volume()
+      np.testing.assert_array_equal(b[key][:off], host[key][:off])
+      rows = lambda x: x[off:off + N * vol].reshape(N, vol)
+      np.testing.assert_array_equal(rows(b[key])[~mask], rows(host[key])[~mask])
+      assert normwise_error(b[key], a[key], vol, off) <= TOL[et.fp_type]
