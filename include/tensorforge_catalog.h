@@ -57,8 +57,42 @@ void launcher_kernel_b042afe2ce(double* m0, unsigned m0_extraOffset, const doubl
 void launcher_kernel_00f28504d5(float* m0, unsigned m0_extraOffset, const float* m1, unsigned m1_extraOffset, const float* m2, size_t numElements, unsigned* flags, void* streamPtr);
 /* inplace_volume_84 */
 void launcher_kernel_db3b423e76(double* m0, unsigned m0_extraOffset, const double* m1, unsigned m1_extraOffset, const double* m2, size_t numElements, unsigned* flags, void* streamPtr);
-/* opt_t_matrix_chain_20x70x20_vector, t_matrix_chain_20x70x20_auto, t_matrix_chain_20x70x20_plain */
+/* matrix_direct_chain_13x6x29_q4, matrix_staged_chain_13x6x29_q4, t_matrix_chain_13x6x29_q4_auto, t_matrix_chain_13x6x29_q4_plain */
+void launcher_kernel_83309835bc(const double* m0, unsigned m0_extraOffset, const double* m1, unsigned m1_extraOffset, const double* m2, double* m3, unsigned m3_extraOffset, const double* m4, size_t numElements, unsigned* flags, void* streamPtr);
+/* matrix_direct_chain_20x70x20, matrix_staged_chain_20x70x20, opt_t_matrix_chain_20x70x20_vector, t_matrix_chain_20x70x20_auto, t_matrix_chain_20x70x20_plain */
 void launcher_kernel_4507257447(const double* m0, unsigned m0_extraOffset, const double* m1, unsigned m1_extraOffset, const double* m2, double* m3, unsigned m3_extraOffset, const double* m4, size_t numElements, unsigned* flags, void* streamPtr);
+/* matrix_direct_chain_37x18x50_f32, matrix_staged_chain_37x18x50_f32, t_matrix_chain_37x18x50_f32_auto, t_matrix_chain_37x18x50_f32_plain */
+void launcher_kernel_3986b41b4e(const float* m0, unsigned m0_extraOffset, const float* m1, unsigned m1_extraOffset, const float* m2, float* m3, unsigned m3_extraOffset, const float* m4, size_t numElements, unsigned* flags, void* streamPtr);
+/* matrix_direct_chain_56x21x56, matrix_staged_chain_56x21x56, t_matrix_chain_56x21x56_auto, t_matrix_chain_56x21x56_plain */
+void launcher_kernel_286f279ee6(const double* m0, unsigned m0_extraOffset, const double* m1, unsigned m1_extraOffset, const double* m2, double* m3, unsigned m3_extraOffset, const double* m4, size_t numElements, unsigned* flags, void* streamPtr);
+/* matrix_direct_gemm_16x16_q1, matrix_staged_gemm_16x16_q1, t_matrix_gemm_16x16_q1_auto, t_matrix_gemm_16x16_q1_plain */
+void launcher_kernel_62a7014a00(double* m0, unsigned m0_extraOffset, const double* m1, const double* m2, unsigned m2_extraOffset, size_t numElements, unsigned* flags, void* streamPtr);
+/* matrix_direct_gemm_18x21_q8, matrix_staged_gemm_18x21_q8, t_matrix_gemm_18x21_q8_auto, t_matrix_gemm_18x21_q8_plain */
+void launcher_kernel_1e872f8b7f(double* m0, unsigned m0_extraOffset, const double* m1, const double* m2, unsigned m2_extraOffset, size_t numElements, unsigned* flags, void* streamPtr);
+/* matrix_direct_gemm_33x35_q10, matrix_staged_gemm_33x35_q10, t_matrix_gemm_33x35_q10_auto, t_matrix_gemm_33x35_q10_plain */
+void launcher_kernel_52fd62987d(double* m0, unsigned m0_extraOffset, const double* m1, const double* m2, unsigned m2_extraOffset, size_t numElements, unsigned* flags, void* streamPtr);
+/* matrix_direct_gemm_50x33_q16_f32, matrix_staged_gemm_50x33_q16_f32, t_matrix_gemm_50x33_q16_f32_auto, t_matrix_gemm_50x33_q16_f32_plain */
+void launcher_kernel_0101b257e7(float* m0, unsigned m0_extraOffset, const float* m1, const float* m2, unsigned m2_extraOffset, size_t numElements, unsigned* flags, void* streamPtr);
+/* matrix_direct_gemm_57x60, matrix_staged_gemm_57x60, t_matrix_gemm_57x60_auto, t_matrix_gemm_57x60_plain */
+void launcher_kernel_a48511a2a0(double* m0, unsigned m0_extraOffset, const double* m1, const double* m2, unsigned m2_extraOffset, size_t numElements, unsigned* flags, void* streamPtr);
+/* matrix_direct_gemm_5x3, matrix_staged_gemm_5x3, t_matrix_gemm_5x3_auto, t_matrix_gemm_5x3_plain */
+void launcher_kernel_c2a08e2d8b(double* m0, unsigned m0_extraOffset, const double* m1, const double* m2, unsigned m2_extraOffset, size_t numElements, unsigned* flags, void* streamPtr);
+/* matrix_direct_gemm_7x5_f32, matrix_staged_gemm_7x5_f32, t_matrix_gemm_7x5_f32_auto, t_matrix_gemm_7x5_f32_plain */
+void launcher_kernel_d47df54798(float* m0, unsigned m0_extraOffset, const float* m1, const float* m2, unsigned m2_extraOffset, size_t numElements, unsigned* flags, void* streamPtr);
+/* matrix_direct_gemm_84x83, matrix_staged_gemm_84x83, t_matrix_gemm_84x83_auto, t_matrix_gemm_84x83_plain */
+void launcher_kernel_d6949a2e25(double* m0, unsigned m0_extraOffset, const double* m1, const double* m2, unsigned m2_extraOffset, size_t numElements, unsigned* flags, void* streamPtr);
+/* matrix_direct_volume_12, matrix_staged_volume_12, t_matrix_volume_12_auto, t_matrix_volume_12_plain */
+void launcher_kernel_df0187eec2(const double* m0, unsigned m0_extraOffset, const double* m1, unsigned m1_extraOffset, double* m2, unsigned m2_extraOffset, const double* m3, size_t numElements, unsigned* flags, void* streamPtr);
+/* matrix_direct_volume_35, matrix_staged_volume_35, t_matrix_volume_35_auto, t_matrix_volume_35_plain */
+void launcher_kernel_86fefd5e47(const double* m0, unsigned m0_extraOffset, const double* m1, unsigned m1_extraOffset, double* m2, unsigned m2_extraOffset, const double* m3, size_t numElements, unsigned* flags, void* streamPtr);
+/* matrix_direct_volume_41x47_q5, matrix_staged_volume_41x47_q5, t_matrix_volume_41x47_q5_auto, t_matrix_volume_41x47_q5_plain */
+void launcher_kernel_f4590f8b42(const double* m0, unsigned m0_extraOffset, const double* m1, unsigned m1_extraOffset, double* m2, unsigned m2_extraOffset, const double* m3, size_t numElements, unsigned* flags, void* streamPtr);
+/* matrix_direct_volume_61x59_f32, matrix_staged_volume_61x59_f32, t_matrix_volume_61x59_f32_auto, t_matrix_volume_61x59_f32_plain */
+void launcher_kernel_187c9a7d18(const float* m0, unsigned m0_extraOffset, const float* m1, unsigned m1_extraOffset, float* m2, unsigned m2_extraOffset, const float* m3, size_t numElements, unsigned* flags, void* streamPtr);
+/* matrix_direct_volume_84x84, matrix_staged_volume_84x84, t_matrix_volume_84x84_auto, t_matrix_volume_84x84_plain */
+void launcher_kernel_11f23039a7(const double* m0, unsigned m0_extraOffset, const double* m1, unsigned m1_extraOffset, double* m2, unsigned m2_extraOffset, const double* m3, size_t numElements, unsigned* flags, void* streamPtr);
+/* matrix_direct_volume_90x30_f32, matrix_staged_volume_90x30_f32, t_matrix_volume_90x30_f32_auto, t_matrix_volume_90x30_f32_plain */
+void launcher_kernel_5319ef52cf(const float* m0, unsigned m0_extraOffset, const float* m1, unsigned m1_extraOffset, float* m2, unsigned m2_extraOffset, const float* m3, size_t numElements, unsigned* flags, void* streamPtr);
 /* pw_clamp_scale_f64 */
 void launcher_kernel_b29a95e19f(double* m0, unsigned m0_extraOffset, double m1, size_t numElements, unsigned* flags, void* streamPtr);
 /* pw_plastic_f64 */
@@ -125,40 +159,6 @@ void launcher_kernel_2a2994fb98(double* m0, unsigned m0_extraOffset, const doubl
 void launcher_kernel_6fedf5eca0(double* m0, unsigned m0_extraOffset, const double* m1, const double* m2, unsigned m2_extraOffset, size_t numElements, unsigned* flags, void* streamPtr);
 /* t_mat_vec_auto, t_mat_vec_plain */
 void launcher_kernel_090c1dade6(float* m0, unsigned m0_extraOffset, const float* m1, unsigned m1_extraOffset, const float* m2, unsigned m2_extraOffset, size_t numElements, unsigned* flags, void* streamPtr);
-/* t_matrix_chain_13x6x29_q4_auto, t_matrix_chain_13x6x29_q4_plain */
-void launcher_kernel_83309835bc(const double* m0, unsigned m0_extraOffset, const double* m1, unsigned m1_extraOffset, const double* m2, double* m3, unsigned m3_extraOffset, const double* m4, size_t numElements, unsigned* flags, void* streamPtr);
-/* t_matrix_chain_37x18x50_f32_auto, t_matrix_chain_37x18x50_f32_plain */
-void launcher_kernel_3986b41b4e(const float* m0, unsigned m0_extraOffset, const float* m1, unsigned m1_extraOffset, const float* m2, float* m3, unsigned m3_extraOffset, const float* m4, size_t numElements, unsigned* flags, void* streamPtr);
-/* t_matrix_chain_56x21x56_auto, t_matrix_chain_56x21x56_plain */
-void launcher_kernel_286f279ee6(const double* m0, unsigned m0_extraOffset, const double* m1, unsigned m1_extraOffset, const double* m2, double* m3, unsigned m3_extraOffset, const double* m4, size_t numElements, unsigned* flags, void* streamPtr);
-/* t_matrix_gemm_16x16_q1_auto, t_matrix_gemm_16x16_q1_plain */
-void launcher_kernel_62a7014a00(double* m0, unsigned m0_extraOffset, const double* m1, const double* m2, unsigned m2_extraOffset, size_t numElements, unsigned* flags, void* streamPtr);
-/* t_matrix_gemm_18x21_q8_auto, t_matrix_gemm_18x21_q8_plain */
-void launcher_kernel_1e872f8b7f(double* m0, unsigned m0_extraOffset, const double* m1, const double* m2, unsigned m2_extraOffset, size_t numElements, unsigned* flags, void* streamPtr);
-/* t_matrix_gemm_33x35_q10_auto, t_matrix_gemm_33x35_q10_plain */
-void launcher_kernel_52fd62987d(double* m0, unsigned m0_extraOffset, const double* m1, const double* m2, unsigned m2_extraOffset, size_t numElements, unsigned* flags, void* streamPtr);
-/* t_matrix_gemm_50x33_q16_f32_auto, t_matrix_gemm_50x33_q16_f32_plain */
-void launcher_kernel_0101b257e7(float* m0, unsigned m0_extraOffset, const float* m1, const float* m2, unsigned m2_extraOffset, size_t numElements, unsigned* flags, void* streamPtr);
-/* t_matrix_gemm_57x60_auto, t_matrix_gemm_57x60_plain */
-void launcher_kernel_a48511a2a0(double* m0, unsigned m0_extraOffset, const double* m1, const double* m2, unsigned m2_extraOffset, size_t numElements, unsigned* flags, void* streamPtr);
-/* t_matrix_gemm_5x3_auto, t_matrix_gemm_5x3_plain */
-void launcher_kernel_c2a08e2d8b(double* m0, unsigned m0_extraOffset, const double* m1, const double* m2, unsigned m2_extraOffset, size_t numElements, unsigned* flags, void* streamPtr);
-/* t_matrix_gemm_7x5_f32_auto, t_matrix_gemm_7x5_f32_plain */
-void launcher_kernel_d47df54798(float* m0, unsigned m0_extraOffset, const float* m1, const float* m2, unsigned m2_extraOffset, size_t numElements, unsigned* flags, void* streamPtr);
-/* t_matrix_gemm_84x83_auto, t_matrix_gemm_84x83_plain */
-void launcher_kernel_d6949a2e25(double* m0, unsigned m0_extraOffset, const double* m1, const double* m2, unsigned m2_extraOffset, size_t numElements, unsigned* flags, void* streamPtr);
-/* t_matrix_volume_12_auto, t_matrix_volume_12_plain */
-void launcher_kernel_df0187eec2(const double* m0, unsigned m0_extraOffset, const double* m1, unsigned m1_extraOffset, double* m2, unsigned m2_extraOffset, const double* m3, size_t numElements, unsigned* flags, void* streamPtr);
-/* t_matrix_volume_35_auto, t_matrix_volume_35_plain */
-void launcher_kernel_86fefd5e47(const double* m0, unsigned m0_extraOffset, const double* m1, unsigned m1_extraOffset, double* m2, unsigned m2_extraOffset, const double* m3, size_t numElements, unsigned* flags, void* streamPtr);
-/* t_matrix_volume_41x47_q5_auto, t_matrix_volume_41x47_q5_plain */
-void launcher_kernel_f4590f8b42(const double* m0, unsigned m0_extraOffset, const double* m1, unsigned m1_extraOffset, double* m2, unsigned m2_extraOffset, const double* m3, size_t numElements, unsigned* flags, void* streamPtr);
-/* t_matrix_volume_61x59_f32_auto, t_matrix_volume_61x59_f32_plain */
-void launcher_kernel_187c9a7d18(const float* m0, unsigned m0_extraOffset, const float* m1, unsigned m1_extraOffset, float* m2, unsigned m2_extraOffset, const float* m3, size_t numElements, unsigned* flags, void* streamPtr);
-/* t_matrix_volume_84x84_auto, t_matrix_volume_84x84_plain */
-void launcher_kernel_11f23039a7(const double* m0, unsigned m0_extraOffset, const double* m1, unsigned m1_extraOffset, double* m2, unsigned m2_extraOffset, const double* m3, size_t numElements, unsigned* flags, void* streamPtr);
-/* t_matrix_volume_90x30_f32_auto, t_matrix_volume_90x30_f32_plain */
-void launcher_kernel_5319ef52cf(const float* m0, unsigned m0_extraOffset, const float* m1, unsigned m1_extraOffset, float* m2, unsigned m2_extraOffset, const float* m3, size_t numElements, unsigned* flags, void* streamPtr);
 /* t_pw_big */
 void launcher_kernel_0ed654b475(double* m0, unsigned m0_extraOffset, const double** m1, unsigned m1_extraOffset, size_t numElements, unsigned* flags, void* streamPtr);
 /* t_pw_math_f32 */

@@ -600,6 +600,10 @@ MATRIX_EDGES = {
 }
 for _tag, _kw in MATRIX_EDGES.items():
   register(f't_matrix_{_tag}_plain')(lambda kw=_kw: _matrix_entry(**kw))
+  for _form in ('staged', 'direct'):
+    # the form by name: the default takes the faster one at these sizes
+    register(f'matrix_{_form}_{_tag}')(
+      lambda kw=_kw, form=_form: _option_entry(_matrix_entry(**kw), dict(stream_matrix=form)))
 
 # sparse shared operands at the edges of the form for few elements: rows and contraction rows per
 # wavefront (4), entries per table batch, columns per wavefront (64)

@@ -177,6 +177,25 @@ def unsupported_reason(program, pl):
   return set_unsupported_reason(program, pl)
 
 
+def term_weights(t, columns):
+  """[(column, [(m, position)])] of term t's stored weights in the columns."""
+  prod = t.producer
+  mlo, mhi = prod.k_ranges[0]
+  c_lo = prod.n_ranges[1][0]
+  rk, rn = t.w_dims
+  out = []
+  for c in columns:
+    ms = []
+    for m in range(mlo, mhi):
+      idx = [0, 0]
+      idx[rk], idx[rn] = m, c_lo + c
+      pos = t.W.packed.get(tuple(idx)) if t.W.is_sparse() else t.W.offset(idx)
+      if pos is not None:
+        ms.append((m, pos))
+    out.append((c, ms))
+  return out
+
+
 class _Tile:
   def __init__(self, program, context, base_name, pl):
     self.prog, self.ctx, self.pl = program, context, pl
@@ -229,22 +248,7 @@ class _Tile:
     return (4 * big + small * (1 if self.f64 else 5)) * (self.size // 4) * len(self.halves[0])
 
   def weights(self, t, half):
-    """[(column, [(m, position)])] of term t's stored weights in the half's columns."""
-    prod = t.producer
-    mlo, mhi = prod.k_ranges[0]
-    c_lo = prod.n_ranges[1][0]
-    rk, rn = t.w_dims
-    out = []
-    for c in half:
-      ms = []
-      for m in range(mlo, mhi):
-        idx = [0, 0]
-        idx[rk], idx[rn] = m, c_lo + c
-        pos = t.W.packed.get(tuple(idx)) if t.W.is_sparse() else t.W.offset(idx)
-        if pos is not None:
-          ms.append((m, pos))
-      out.append((c, ms))
-    return out
+    return term_weights(t, half)
 
   def weight_span(self, t, half):
     ps = [p for _, ms in self.weights(t, half) for _, p in ms]
@@ -942,20 +946,54 @@ def set_times(program, pl):
   return memory, total * pl.q / 4 / 2200.0
 
 
-def staged_pays(program, pl):
-  """The staged form moves whole lines but separates a set's steps by barriers: it is the faster
-  one where memory time is the longer and a set is large enough (C += A B over 800 MB: 10 to 84
-  rows 210-295 us against 271-295, flux integral over 131,072 elements 337 against 424); the
-  volume chain has as much matrix time as memory time from 35 rows up and less than 64 KB per set
-  below (35 rows 306 us direct, 399 staged; 20 rows 103 and 134)."""
-  memory, matrix = set_times(program, pl)
+def forms(program, pl):
+  """The matrix-core forms that are faster than the vector stream, the fastest first: of 'staged'
+  and 'direct'. Measured on 400 MB of operands, times in us.
+
+  The staged form moves whole lines, but a set's steps are separated by barriers: it needs enough
+  bytes per set of 16 elements, the more the better the vector stream's lanes use the lines of
+  their columns. C += A B (vector / staged), columns of 112 bytes and more: 16 KB sets 97 / 95, 18 KB
+  102 / 89, 9 KB 103 / 124; of 64 to 96 bytes: 18 KB 91 / 88, 12 KB 86 / 104; below: 36 KB 84 / 80,
+  30 KB 84 / 94, 9 KB 80 / 122. Where a set is smaller the direct form is faster for columns of
+  whole lines (16 x 16 FP64, one column: 99 / 84; 32 x 32 FP32, two columns: 100 / 86), but not for
+  shorter ones (4 to 12 rows, two columns: 77-91 / 90-105).
+
+  Flux chains: 32 KB sets 103 direct / 80 staged, 22 KB FP32 99 vector / 91 staged, 16 KB 98 / 99.
+  A chain of one shared operand per term is staged where memory time is as long as matrix time (35
+  rows 171 direct / 160 staged, 40 rows 156 / 158), a set has 64 KB (55 KB 113 / 116) and its
+  wavefronts form little more than the stored products: one quantity each and a share of a ninth
+  (16 columns, 10 rows: 138 vector / 123 direct / 194 staged), with about as many weights in every
+  column (28 rows, at most 5 weights in a column, 2.7 on average: 136 / 114 / 158; 3 in every
+  column: 137 / 131 / 116).
+
+  The direct form of a chain needs blocks of rows to work on: FP32 blocks have 16 rows (14 rows 127
+  vector / 134 direct, 16 rows 129 / 111, flux chain 10 x 6 rows, three columns 87 / 141), FP64
+  ones 8 (4 rows, one column 79 / 98, nine columns 117 / 113; 6 rows 117 / 109). Of flux chains it
+  holds two products' accumulators (56 x 21 rows FP64, 10 columns 111 / 109, 13 columns 118 / 129,
+  16 columns 127 / 193)."""
+  per_set = element_traffic(program).per_element * SET
+  size = program.fp_type.size()
+  stages = [t.product for t in pl.terms] + [s.product for s in pl.post]
+  extents = [hi - lo for p in stages for lo, hi in (p.n_ranges[0], p.k_ranges[0])]
+  few = min(extents)
   if pl.terms[0].kind == 'global':
-    return True
-  return memory >= matrix and element_traffic(program).per_element * SET >= 64 * 1024
+    column = max(extents) * size
+    if per_set >= (13.5 if column >= 112 else 17 if column >= 64 else 32) * 1024:
+      return ['staged', 'direct']
+    return ['direct'] if few * size >= 128 else []
+  whole = few >= 16 if size == 4 else few >= 6 or per_set >= 16 * 1024
+  if pl.post:
+    return ['staged'] * (per_set >= 20 * 1024) + ['direct'] * (whole and pl.q <= WAVES + 1)
+  memory, matrix = set_times(program, pl)
+  stored = [[len(ms) for _, ms in term_weights(t, range(pl.q))] for t in pl.terms]
+  padded = sum(max(n) * pl.q for n in stored)
+  staged = memory >= 0.95 * matrix and per_set >= 64 * 1024 and pl.q <= WAVES + 1 and \
+      padded <= 1.2 * sum(map(sum, stored))
+  return ['staged'] * staged + ['direct'] * whole
 
 
-def emit(program, context, base_name, pl):
-  """(Emitted, None) or (None, reason)."""
+def emit(program, context, base_name, pl, matrix='auto'):
+  """(Emitted, None) or (None, reason). ``matrix``: 'auto', or the form to take."""
   # a flux chain's plan names its streamed operand once
   pl = replace(pl, terms=[replace(t, L=t.L or pl.L, l_cols=t.l_cols or pl.l_cols)
                           for t in pl.terms])
@@ -963,8 +1001,11 @@ def emit(program, context, base_name, pl):
   if reason is not None:
     return None, reason
   from .staged import _Staged
-  em = None
-  if staged_pays(program, pl):
-    em = _Staged(program, context, base_name, pl).emit()
-  em = em or _Tile(program, context, base_name, pl).emit()
-  return (em, None) if em is not None else (None, 'accumulators or shared operands do not fit')
+  chosen = forms(program, pl) if matrix == 'auto' else [matrix]
+  if not chosen:
+    return None, 'the vector stream is faster'
+  for form in chosen:
+    em = (_Staged if form == 'staged' else _Tile)(program, context, base_name, pl).emit()
+    if em is not None:
+      return em, None
+  return None, 'accumulators or shared operands do not fit'

@@ -97,9 +97,10 @@ class Schedule:
   # blocks (prefetch distance = slots - 1)
   stream_dma: bool = False
   stream_dma_slots: int = 3
-  # matrix-core form of the streaming schedule where the chain admits it (dense shared operands):
-  # 'auto' or 'never'. Without an explicit schedule it is the default; the knobs above describe
-  # the vector form, so an explicit schedule keeps that one
+  # matrix-core form of the streaming schedule (dense shared operands): 'auto' takes the fastest
+  # form by the chain's sizes (tile.forms), 'staged' and 'direct' that one where the chain admits
+  # it, 'never' none. Without an explicit schedule it is 'auto'; the knobs above describe the vector
+  # form, so an explicit schedule keeps that one
   stream_matrix: str = 'never'
   # how the DPP broadcast is issued: 'asm' (one v_fmac_*_dpp) or 'builtin' (v_mov_*_dpp + fma)
   dpp: str = 'asm'
@@ -877,8 +878,8 @@ def emit(program, context, base_name, schedule=None) -> Emitted:
   schedule = schedule or Schedule(stream_matrix='auto')
   if schedule.stream:
     pl, _ = stream.plan(program)
-    if pl is not None and schedule.stream_matrix == 'auto':
-      emitted, _ = tile.emit(program, context, base_name, pl)
+    if pl is not None and schedule.stream_matrix != 'never':
+      emitted, _ = tile.emit(program, context, base_name, pl, schedule.stream_matrix)
       if emitted is not None:
         return emitted
     if pl is not None:

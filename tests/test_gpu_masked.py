@@ -1,6 +1,6 @@
 """Masked launches and extra offsets through the matrix-core and vector forms of both types.
 
-60,001 elements (several rounds of a workgroup, a partial last set), every per-element operand behind
+20,011 elements (more than one round of a workgroup, a partial last set), every per-element operand behind
 an odd number of unused entries, masks that skip single elements, whole sets of 16 and everything;
 every element is compared with the plain launcher of the same chain. Normwise per element 1e-12
 FP64, 1e-5 FP32.
@@ -14,8 +14,9 @@ from harness import TOL, gpu_run, key_of, make_inputs, normwise_error, outputs_o
 
 pytestmark = pytest.mark.gpu
 
-N = 60001
+N = 20011
 MASKS = {
+  'all': np.ones(N, bool),
   'single': np.arange(N) % 5 != 3,
   'runs': np.arange(N) // 37 % 3 == 1,
   'few': np.arange(N) % 1013 == 7,
@@ -24,13 +25,15 @@ MASKS = {
 ENTRIES = ['ader_f32_tuned', 'ader_dense_f64_tuned', 'ader_dense_f32_tuned', 'ader7_f64_tuned',
            'gemm_f64_tuned', 'gemm_f32_tuned', 'flux_local_mod_f64_tuned',
            'flux_neigh_mod_f64_tuned', 'deriv_f64_tuned', 'deriv_na_f64_tuned']
-ENTRIES += [f't_matrix_{t}_auto' for t in catalog.MATRIX_EDGES]
+PLAIN = {name: name.rsplit('_', 1)[0] + '_plain' for name in ENTRIES}
+PLAIN.update({f'matrix_{form}_{t}': f't_matrix_{t}_plain' for form in ('staged', 'direct')
+              for t in catalog.MATRIX_EDGES})
 
 
-@pytest.mark.parametrize('name', ENTRIES)
+@pytest.mark.parametrize('name', list(PLAIN))
 def test_masked_with_offsets(name, device):
   et, kt = catalog.load(name)
-  ep, kp = catalog.load(name.rsplit('_', 1)[0] + '_plain')
+  ep, kp = catalog.load(PLAIN[name])
   keys = [key_of(t) for t in ep.generator._global_tensors if t.addressing.name == 'STRIDED']
   offsets = {k: 3 + 2 * i for i, k in enumerate(keys)}
   host = make_inputs(ep, N, seed=29, offsets=offsets)
