@@ -30,6 +30,7 @@ from .traffic import element_traffic
 
 WAVE = 64
 CHUNK = 16
+LDS_LIMIT = 160 * 1024
 
 
 @dataclass
@@ -429,8 +430,13 @@ class _Stream:
     # the groups of a workgroup are taken by its wavefronts as they get to them: of two wavefronts
     # on a SIMD the older one is served first, and with fixed shares it ends early (48,000 cycles a
     # group against 65,000, order-6 volume chain FP64) and leaves the other one alone (262,144
-    # elements 699 us, now 691; FP32, 200,000 elements 329, now 318)
-    claims = not self.loop and not self.dma
+    # elements 699 us, now 691; FP32, 200,000 elements 329, now 318). A chain that waits for memory
+    # pays for reads that spread over more lines: FP64 ones take their groups so where they have
+    # work for their bytes (800 MB, fixed / taken: volume chains of 28 rows 233 / 240 us, 48 rows 246 /
+    # 249, 64 rows 258 / 255, 84 rows 326 / 319; GEMM with statements 211 / 219), FP32 ones always
+    # (volume chains of 10 to 84 rows 237-443 / 229-419, GEMMs 168-252 / 165-249)
+    claims = not self.loop and not self.dma and lds_bytes + 32 <= LDS_LIMIT and \
+        (self.fp == FloatingPointType.FLOAT or self.busy())
     if claims:
       lds_bytes = (lds_bytes + 15) // 16 * 16 + 16
     # tables: position of every traversal entry in its U array, term in the top bits
@@ -611,6 +617,12 @@ class _Stream:
           self.offsets[ms] = o
         entries.append((v, self.offsets[ms]))
       self.slots[t_idx] = entries
+
+  def busy(self):
+    """The chain has work for its bytes: 25 multiply-adds and more for each entry moved (sparse
+    volume chains of 48 rows and more, 31 at order 6)."""
+    moved = element_traffic(self.prog).per_element / self.fp.size()
+    return self.nu * self.q >= 25 * moved
 
   def early_weights(self):
     """The next group's weights are loaded before this group's results are stored. Loaded at the
