@@ -627,9 +627,19 @@ class _Stream:
   def early_weights(self):
     """The next group's weights are loaded before this group's results are stored. Loaded at the
     top of the group they would wait for those stores: the memory counter is in order (order-6
-    volume chain FP32, 200,000 elements 356 us so, 329 now; FP64, 262,144 elements 705 / 699)."""
-    return bool(self.slots) and not self.loop and not self.dma and \
-        all(t.W.arg.addressing == Addressing.STRIDED for t in self.pl.terms if t.kind == 'fused')
+    volume chain FP32, 200,000 elements 356 us so, 329 now; FP64, 262,144 elements 705 / 699). They
+    are read twice (a line each ahead of time) and stay in registers, which chains that wait for
+    memory or hold many weights in FP64 pay for (800 MB, at the top / early: volume chains FP64 of
+    12 rows 230 / 241 us, 35 rows 261 / 273, 64 rows 255 / 248, 84 rows 319 / 310, 56 rows with 27
+    weights a column 262 / 295; FP32 35 rows 270 / 284, 56 rows 283 / 273, 20 rows with 27 weights
+    a column 228 / 212)."""
+    if not self.slots or self.loop or self.dma or \
+        any(t.W.arg.addressing != Addressing.STRIDED for t in self.pl.terms if t.kind == 'fused'):
+      return False
+    held = sum(map(len, self.slots.values()))
+    if self.fp == FloatingPointType.FLOAT and held >= 16:
+      return True
+    return self.busy() and held * self.fp.size() // 4 <= 32
 
   def weights(self, pointer, declare=''):
     """Weights of the fused temporaries; their positions are recomputed from an opaque copy of

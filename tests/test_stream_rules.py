@@ -1,5 +1,5 @@
-"""Where the vector stream's wavefronts take their groups as they get to them: by work per entry
-moved and type."""
+"""Where the vector stream's wavefronts take their groups as they get to them and where the next
+group's weights are loaded early: by work per entry moved, type and weights held."""
 import pytest
 
 from tensorforge_amd import catalog
@@ -16,28 +16,28 @@ def _rules(g):
   g.generate()
   src, lds = g.get_emitted().kernel_src, g.get_emitted().lds_bytes
   assert lds <= stream.LDS_LIMIT
-  return 'fetch_add(claim' in src
+  return 'fetch_add(claim' in src, 'const size_t ew =' in src
 
 
-@pytest.mark.parametrize('fp, b, claims', [
-  (F64, 10, False), (F64, 35, False), (F64, 56, True), (F64, 84, True),
-  (F32, 10, True), (F32, 35, True), (F32, 56, True)])
-def test_volume(fp, b, claims):
+@pytest.mark.parametrize('fp, b, claims, early', [
+  (F64, 10, False, False), (F64, 35, False, False), (F64, 56, True, True), (F64, 84, True, True),
+  (F32, 10, True, False), (F32, 35, True, False), (F32, 56, True, True)])
+def test_volume(fp, b, claims, early):
   g = Generator(W.ader_volume(fp, b=b).descrs, Context('gfx950', 'hip', fp))
-  assert _rules(g) == claims
+  assert _rules(g) == (claims, early)
 
 
-@pytest.mark.parametrize('fp, m, claims', [
-  (F64, 57, False), (F32, 20, True)])
-def test_one_term(fp, m, claims):
+@pytest.mark.parametrize('fp, m, claims, early', [
+  (F64, 57, False, False), (F32, 20, True, False)])
+def test_one_term(fp, m, claims, early):
   for dense in (False, True):
     e = catalog._matrix_entry('volume', m=m, k=m, q=9, fp=fp, dense_star=dense, sparse=True)
-    assert _rules(Generator(e.descrs, Context('gfx950', 'hip', fp))) == claims
+    assert _rules(Generator(e.descrs, Context('gfx950', 'hip', fp))) == (claims, early)
 
 
 def test_gemm_with_statements():
   e = catalog.get('t_fused_gemm_pw')
-  assert not _rules(e.generator)
+  assert _rules(e.generator) == (False, False)
 
 
 def test_both_ways_in_one_grouped_launch():
