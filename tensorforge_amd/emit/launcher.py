@@ -39,9 +39,14 @@ class Emitted:
   # a kernel of the same chain for launches of at most ``few_limit`` elements
   few: 'Emitted' = None
   few_limit: int = 0
+  # a kernel of the same chain for launches with flags of more than ``masked_from`` elements per
+  # compute unit
+  masked: 'Emitted' = None
+  masked_from: int = 0
 
   def full_source(self):
-    return self.kernel_src + ''.join(e.full_source() for e in (self.fallback, self.few) if e)
+    return self.kernel_src + ''.join(e.full_source()
+                                     for e in (self.fallback, self.few, self.masked) if e)
 
 
 class Writer:
@@ -179,6 +184,12 @@ def launcher_source(generator, emitted: Emitted) -> str:
       with w.block(f'if ({GeneralLexicon.NUM_ELEMENTS} <= {emitted.few_limit})'):
         _launch_block(w, generator, emitted.few)
         w('return;')
+    if emitted.masked is not None:
+      w.lines(COMPUTE_UNITS)
+      with w.block(f'if (flags != nullptr && {GeneralLexicon.NUM_ELEMENTS} > '
+                   f'{emitted.masked_from}ull * tf_cus)'):
+        _launch_block(w, generator, emitted.masked)
+        w('return;')
     if emitted.fallback is not None:
       with w.block(f'if ({emitted.condition})'):
         _launch_block(w, generator, emitted)
@@ -187,6 +198,17 @@ def launcher_source(generator, emitted: Emitted) -> str:
     else:
       _launch_block(w, generator, emitted)
   return w.src()
+
+
+# compute units of the device (queried once; 0 if that fails: the launch that follows reports it)
+COMPUTE_UNITS = '''static int tf_cus = 0;
+if (tf_cus == 0) {
+  int dev = 0, cus = 0;
+  if (hipGetDevice(&dev) != hipSuccess ||
+      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
+    (void)hipGetLastError();
+  tf_cus = cus;
+}'''
 
 
 def _launch_block(w, generator, emitted):
@@ -268,12 +290,13 @@ def distinct_symbol(emitted: Emitted) -> Emitted:
   new = f'{old}_{form}_{digest}'
 
   def rename(em):
-    fb, few = (rename(e) if e is not None else None for e in (em.fallback, em.few))
+    fb, few, masked = (rename(e) if e is not None else None
+                       for e in (em.fallback, em.few, em.masked))
     return dataclasses.replace(em, kernel_name=em.kernel_name.replace(old, new),
                                kernel_src=em.kernel_src.replace(old, new),
                                extra_launch_setup=em.extra_launch_setup.replace(old, new),
                                condition=em.condition.replace(old, new), fallback=fb,
-                               few=few)
+                               few=few, masked=masked)
   return rename(emitted)
 
 

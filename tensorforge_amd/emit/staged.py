@@ -48,6 +48,7 @@ class _Pieces:
   def __init__(self, tag, arg, rows, cols, first, col_stride, lds_rows, lds_elem, lds_base, per,
                lds_run=None, elements=SET, threads=THREADS):
     self.tag, self.arg, self.rows, self.elements = tag, arg, rows, elements
+    self.listed = False          # the set's elements come from a list: no distance between them
     self.first, self.col_stride = first, col_stride      # storage offset of run 0, of the next run
     self.lds_elem, self.lds_base = lds_elem, lds_base
     self.lds_run = lds_run or lds_rows                   # distance of two runs in LDS
@@ -108,7 +109,8 @@ class _Pieces:
     if self.moved:
       w(f'{t}h = pp > {self.rows - self.per} ? pp - {self.rows - self.per} : 0;')
       sh = f' - {t}h'
-    w(f'{t}g = {t}e * {self.arg.element_stride} + {self.first} + pm * {self.col_stride} + pp{sh};')
+    e = '' if self.listed else f'{t}e * {self.arg.element_stride} + '
+    w(f'{t}g = {e}{self.first} + pm * {self.col_stride} + pp{sh};')
     w(f'{t}l = {self.lds_base} + {t}e * {self.lds_elem} + pm * {self.lds_run} + pp;')
 
   def each(self, w, body):
@@ -123,7 +125,8 @@ class _Pieces:
         body(n)
 
   def at(self, j, bp='bp'):
-    return f'{bp} + {j * self.step * self.arg.element_stride} + {self.tag}g'
+    step = 0 if self.listed else j * self.step * self.arg.element_stride
+    return f'{bp} + {step} + {self.tag}g'
 
   def lds(self, j):
     return f'lds + {self.tag}l + {j * self.step * self.lds_elem}'
@@ -136,7 +139,16 @@ class _SetKernel:
   """A workgroup's loop over sets of ``elements`` elements: the way of the operands and results
   between memory, registers and LDS. A form supplies its geometry (``xstage`` and ``wstage`` per
   phase, ``out``, ``dest``, ``old_early``) and ``place``, ``shared``, ``acc_declare``, ``compute``,
-  ``results``."""
+  ``results``.
+
+  ``masked``: the kernel for launches with flags. It takes the same sets, 32 at a time, lists their
+  active elements in LDS and forms sets of 16 from the list: masked elements are neither moved nor
+  multiplied (an element's run is some KB, so whole lines remain). Vector form / sets of masked and
+  active elements / this one: neighbour flux integral, 40,001 elements, every fourth masked 126 / 121
+  / 102 us, nine tenths masked 86 / 114 / 29; C += A B, 65,536 elements 186 / 142 / 117 and 109 / 123 /
+  32; derivative step, 131,071 elements 613 / 549 / 437 and 517 / 537 / 99. Where flags mask nothing the
+  list costs 2-4 % (558 / 580 us)."""
+  masked = False
 
   def barrier(self):
     # this wavefront's LDS accesses done, every wavefront here; memory accesses stay in flight
@@ -151,7 +163,6 @@ class _SetKernel:
       for _, _, _, p in stage:
         p.declare(w)
     self.out.declare(w)
-    w(f'const size_t nsets = (numElements + {self.elements - 1}) / {self.elements};')
     beta = self.beta_load()
     vt = self.lds_t
     n = max(x.count for x in self.xstage)
@@ -165,39 +176,104 @@ class _SetKernel:
     if beta is not None and not self.old_early:
       touches = [f'touched{j}' for j in range(self.touches())]
       w(f'unsigned {", ".join(touches)};')
+    if self.masked:
+      self.shared()
+      w(f'const size_t every = (numElements + {SET - 1}) / {SET};')
+      with w.block(f'for (size_t first = blockIdx.x; first < every; '
+                   f'first += {THREADS // SET}ull * gridDim.x)'):
+        self.scan()
+        w('if (nsets == 0) continue;')
+        w('int set = 0;')
+        self.fetch(0, 'set')
+        self.arrived()
+        with w.block('for (; set < nsets; ++set)'):
+          self.one_set(beta, touches, 'set + 1')
+      return
+    w(f'const size_t nsets = (numElements + {self.elements - 1}) / {self.elements};')
     w('size_t set = blockIdx.x;')
     # the first set's operands are on their way while the shared ones are staged
     self.fetch(0, 'set')
     self.shared()
     self.arrived()
     with w.block('for (; set < nsets; set += gridDim.x)'):
-      self.acc_declare()
-      for pi, ph in enumerate(self.phases):
-        self.put(pi)
-        self.barrier()
-        last = pi == len(self.phases) - 1
-        if last:
+      self.one_set(beta, touches, 'set + gridDim.x')
+
+  def one_set(self, beta, touches, following):
+    w = self.w
+    self.acc_declare()
+    for pi, ph in enumerate(self.phases):
+      self.put(pi)
+      self.barrier()
+      last = pi == len(self.phases) - 1
+      if last:
+        if not self.masked:
           self.mask_load()
-          if beta is not None and self.old_early:
-            self.move(self.out, 'dv', 'set')
-          elif beta is not None:
-            self.touch()
-          with w.block('if (set + gridDim.x < nsets)'):
-            self.fetch(0, '(set + gridDim.x)')
-        else:
-          self.fetch(pi + 1, 'set')
-        self.compute(pi)
-        self.barrier()
-      self.results()
+        if beta is not None and self.old_early:
+          self.move(self.out, 'dv', 'set')
+        elif beta is not None:
+          self.touch()
+        with w.block(f'if ({following} < nsets)'):
+          self.fetch(0, f'({following})')
+      else:
+        self.fetch(pi + 1, 'set')
+      self.compute(pi)
       self.barrier()
-      if touches:
-        w(f'asm volatile("" :: {", ".join(f"{chr(34)}v{chr(34)}({t})" for t in touches)});')
-        self.move(self.out, 'dv', 'set')
-      # the next set's operands have arrived before the results are stored: waiting for them
-      # afterwards would wait for the stores as well
-      self.arrived()
-      self.leave(beta)
-      self.barrier()
+    self.results()
+    self.barrier()
+    if touches:
+      w(f'asm volatile("" :: {", ".join(f"{chr(34)}v{chr(34)}({t})" for t in touches)});')
+      self.move(self.out, 'dv', 'set')
+    # the next set's operands have arrived before the results are stored: waiting for them
+    # afterwards would wait for the stores as well
+    self.arrived()
+    self.leave(beta)
+    self.barrier()
+
+  # ------------------------------------------------------------------ active elements
+  def list_bytes(self):
+    return 2 * THREADS + 4 * WAVES
+
+  def scan(self):
+    """Lists the active elements of sets ``first``, ``first + gridDim.x``, ... in LDS: a thread's
+    number is its place in these sets."""
+    w = self.w
+    w('{')
+    w._depth += 1
+    w(f'const size_t e = (first + threadIdx.x / {SET} * (size_t)gridDim.x) * {SET} + '
+      f'threadIdx.x % {SET};')
+    w('const bool on = e < numElements && flags[e] != 0u;')
+    w('const unsigned long long ons = __ballot(on);')
+    w('if (lane == 0) counts[wave] = __popcll(ons);')
+    self.barrier()
+    w('int at = __popcll(ons & ((1ull << lane) - 1ull));')
+    w('listed = 0;')
+    with w.block(f'for (int i = 0; i < {WAVES}; ++i)'):
+      w('at += i < wave ? counts[i] : 0;')
+      w('listed += counts[i];')
+    w('if (on) list[at] = (unsigned short)threadIdx.x;')
+    self.barrier()
+    w('listed = __builtin_amdgcn_readfirstlane(listed);')
+    w._depth -= 1
+    w('}')
+    w(f'const int nsets = (listed + {SET - 1}) / {SET};')
+
+  def list_declare(self, base):
+    """``base``: byte offset of the list in LDS."""
+    w = self.w
+    w(f'unsigned short* list = reinterpret_cast<unsigned short*>(lds) + {base // 2};')
+    w(f'int* counts = reinterpret_cast<int*>(lds) + {(base + 2 * THREADS) // 4};')
+    w('int listed;')
+
+  def element_place(self, name, setexpr, slot):
+    """``name``: the list's entry of a set's ``slot``, past the end its last one. The entries of all
+    pieces are read before the first is used: one LDS latency for all of them."""
+    at = f'{setexpr} * {SET} + {slot}'
+    self.w(f'const int {name} = list[{at} < listed ? {at} : listed - 1];')
+
+  def element_pointer(self, name, arg, place, const=''):
+    self.w(f'{const}{self.real}* __restrict__ {name} = {arg.name} + ((first + ({place} >> 4) * '
+           f'(size_t)gridDim.x) * {SET} + ({place} & 15)) * {arg.element_stride}ull + '
+           f'{arg.name}_extraOffset;')
 
   # ------------------------------------------------------------------ memory <-> registers <-> LDS
   def arrived(self):
@@ -216,6 +292,19 @@ class _SetKernel:
     end = o.first + (self.q - 1) * o.col_stride + o.rows        # of an element's window
     w('{')
     w._depth += 1
+    if self.masked:
+      lines = self.element_lines()
+      for j in range(self.touches()):
+        w(f'const int slot{j} = ((int)threadIdx.x + {j * THREADS}) / {lines};')
+        w(f'const int line{j} = {o.first} + ((int)threadIdx.x + {j * THREADS} - slot{j} * {lines}) '
+          f'* {per};')
+        self.element_place(f'tc{j}', 'set', f'slot{j}')
+        self.element_pointer(f'tp{j}', o.arg, f'tc{j}', 'const ')
+        w(f'touched{j} = *reinterpret_cast<const unsigned*>(tp{j} + (line{j} < {end - 1} ? '
+          f'line{j} : {end - 1}));')
+      w._depth -= 1
+      w('}')
+      return
     w(f'const size_t left = numElements - set * {self.elements};')
     w(f'const int last = ((left < {self.elements} ? (int)left : {self.elements}) - 1) * '
       f'{o.arg.element_stride} + {end - 1};')
@@ -227,7 +316,13 @@ class _SetKernel:
     w._depth -= 1
     w('}')
 
+  def element_lines(self):
+    o = self.out
+    return _ceil((self.q - 1) * o.col_stride + o.rows, 128 // self.size) + 1
+
   def touches(self):
+    if self.masked:
+      return _ceil(self.elements * self.element_lines(), THREADS)
     return _ceil(self.elements * self.dest.element_stride, 128 // self.size * THREADS)
 
   def mask_load(self):
@@ -240,6 +335,10 @@ class _SetKernel:
 
   def mask(self):
     """Bit e: element e of the set is to be stored."""
+    if self.masked:
+      self.w(f'const unsigned live = listed - set * {SET} >= {SET} ? {(1 << SET) - 1}u : '
+             f'(1u << (listed - set * {SET})) - 1u;')
+      return
     self.w(f'const unsigned long long live = __ballot(lane < {self.elements} && '
            f'set * {self.elements} + lane < numElements && (flags == nullptr || fv != 0u));')
 
@@ -250,6 +349,18 @@ class _SetKernel:
     vt = self.vec_t[self.per]
     w('{')
     w._depth += 1
+    if self.masked:
+      x.setup(w)
+      for j in range(x.count):
+        self.element_place(f'c{j}', setexpr, x.element(j))
+      for j in range(x.count):
+        with w.block(''):
+          self.element_pointer(bp, x.arg, f'c{j}', 'const ')
+          w(f'{name}{first + j} = __builtin_nontemporal_load(reinterpret_cast<const {vt}*>('
+            f'{x.at(j, bp)}));')
+      w._depth -= 1
+      w('}')
+      return
     w(f'const {self.real}* __restrict__ {bp} = {x.arg.name} + {setexpr} * '
       f'{self.elements * x.arg.element_stride}ull + {x.arg.name}_extraOffset;')
     w(f'const size_t left = numElements - {setexpr} * {self.elements};')
@@ -312,8 +423,9 @@ class _SetKernel:
     vt = self.vec_t[self.per]
     o.setup(w)
     scale = '' if beta in (None, 1.0) else f'{self.fp.literal(beta)} * '
-    w(f'{self.real}* __restrict__ bp = {o.arg.name} + set * '
-      f'{self.elements * o.arg.element_stride}ull + {o.arg.name}_extraOffset;')
+    if not self.masked:
+      w(f'{self.real}* __restrict__ bp = {o.arg.name} + set * '
+        f'{self.elements * o.arg.element_stride}ull + {o.arg.name}_extraOffset;')
 
     if self.shared_last:
       # the thread's place in the other shares of the last quantity
@@ -321,6 +433,8 @@ class _SetKernel:
       w(f'const {self.real}* sp = lds + {self.share_base} + de * {self.share_elem} + sl;')
 
     def write(j):
+      if self.masked:
+        self.element_pointer('bp', o.arg, f'c{j}')
       if o.aligned:
         w(f'{self.lds_t} rv = *reinterpret_cast<const {self.lds_t}*>({o.lds(j)});')
       else:
@@ -356,6 +470,9 @@ class _SetKernel:
       return run
 
     self.mask()
+    if self.masked:
+      for j in range(o.count):
+        self.element_place(f'c{j}', 'set', o.element(j))
     with w.block(f'if (live == {(1 << self.elements) - 1}ull)'):
       o.each(w, scoped(write))
     with w.block('else'):
@@ -364,6 +481,12 @@ class _SetKernel:
 
 class _Staged(_SetKernel, _Tile):
   elements = SET
+
+  def __init__(self, program, context, base_name, pl, masked=False):
+    super().__init__(program, context, base_name, pl)
+    self.masked = masked
+    if masked:
+      self.kname += '_m'
 
   def prepare(self):
     """Geometry; False when the chain does not fit this form."""
@@ -440,6 +563,11 @@ class _Staged(_SetKernel, _Tile):
     self.tiled_last = self.extra == 1 and not self.post and not self.fused
     if self.shared_last:
       self.lds_bytes = max(self.lds_bytes, end)
+    self.list_base = self.lds_bytes
+    if self.masked:
+      self.lds_bytes += self.list_bytes()
+      if self.lds_bytes > LDS_LIMIT:
+        return False
     cols = 1 if self.extra == 0 or self.shared_last or self.tiled_last else 2
     acc = max((4 * self.tiles(s.dr)[0] + self.tiles(s.dr)[1] * (1 if self.f64 else 5))
               for s in self.stages + self.post)
@@ -467,6 +595,7 @@ class _Staged(_SetKernel, _Tile):
     # the destination's 578; three arrays, 50,000 elements, 278 / 252 / 259 us; flux integral, three
     # arrays here, all 331 us, none 345)
     for p in pieces:
+      p.listed = self.masked
       p.held = len(pieces) <= 3 or (p is self.out and len(self.phases) == 1)
     self.weights_held = 2 if use + slots <= 256 else 1
     return use <= 256
@@ -548,6 +677,8 @@ class _Staged(_SetKernel, _Tile):
     w('const int g = lane / 16;')
     w(f'const {real}* __restrict__ ka = ubuf + lane;')
     w(f'const {real}* __restrict__ ks = ubuf + (lane % 4 + 4 * g);')
+    if self.masked:
+      self.list_declare(self.list_base)
 
   def shared(self):
     for s in self.stages + self.post:

@@ -51,3 +51,23 @@ def test_masked_with_offsets(name, device):
       rows = lambda x: x[off:off + N * vol].reshape(N, vol)
       np.testing.assert_array_equal(rows(b[key])[~mask], rows(host[key])[~mask])
       assert normwise_error(b[key], a[key], vol, off) <= TOL[et.fp_type]
+
+
+@pytest.mark.parametrize('tag', ['gemm_16x16_q1', 'gemm_18x21_q8', 'gemm_7x5_f32', 'chain_13x6x29_q4'])
+def test_more_sets_than_a_list_holds(tag, device):
+  """A workgroup lists the active elements of 32 sets at a time."""
+  n = 500003
+  et, kt = catalog.load(f'matrix_staged_{tag}')
+  ep, kp = catalog.load(f't_matrix_{tag}_plain')
+  host = make_inputs(ep, n, seed=31)
+  for mask in (np.arange(n) % 3 != 1, np.arange(n) // 5000 % 7 == 2, np.arange(n) == n - 1):
+    flags = mask.astype(np.uint32)
+    a = gpu_run(kp, ep, host, n, device, flags=flags)
+    b = gpu_run(kt, et, host, n, device, flags=flags)
+    for t in ep.generator._global_tensors:
+      key = key_of(t)
+      if key not in outputs_of(ep):
+        continue
+      rows = lambda x: x.reshape(n, t.get_real_volume())
+      np.testing.assert_array_equal(rows(b[key])[~mask], rows(host[key])[~mask])
+      assert normwise_error(b[key], a[key], t.get_real_volume()) <= TOL[et.fp_type]
