@@ -36,13 +36,19 @@ class Emitted:
   # launcher's parameters) is false
   fallback: 'Emitted' = None
   condition: str = ''
-  # a kernel of the same chain for launches of at most ``few_limit`` elements
+  # a kernel of the same chain for launches of at most ``few_groups`` of its element groups per
+  # compute unit
   few: 'Emitted' = None
-  few_limit: int = 0
+  few_groups: int = 0
   # a kernel of the same chain for launches with flags of more than ``masked_from`` elements per
   # compute unit
   masked: 'Emitted' = None
   masked_from: int = 0
+
+  @property
+  def few_limit(self):
+    """Largest launch of the kernel for few elements on 256 compute units."""
+    return self.few_groups * 256 * self.few.elements_per_block if self.few else 0
 
   def full_source(self):
     return self.kernel_src + ''.join(e.full_source()
@@ -180,12 +186,14 @@ def launcher_source(generator, emitted: Emitted) -> str:
     w(f'if ({GeneralLexicon.NUM_ELEMENTS} == 0) return;')
     w(f'hipStream_t stream = ({GeneralLexicon.STREAM_PTR_STR} != nullptr) ? '
       f'static_cast<hipStream_t>({GeneralLexicon.STREAM_PTR_STR}) : 0;')
+    if emitted.few is not None or emitted.masked is not None:
+      w.lines(COMPUTE_UNITS)
     if emitted.few is not None:
-      with w.block(f'if ({GeneralLexicon.NUM_ELEMENTS} <= {emitted.few_limit})'):
+      with w.block(f'if ({GeneralLexicon.NUM_ELEMENTS} <= '
+                   f'{emitted.few_groups * emitted.few.elements_per_block}ull * tf_cus)'):
         _launch_block(w, generator, emitted.few)
         w('return;')
     if emitted.masked is not None:
-      w.lines(COMPUTE_UNITS)
       with w.block(f'if (flags != nullptr && {GeneralLexicon.NUM_ELEMENTS} > '
                    f'{emitted.masked_from}ull * tf_cus)'):
         _launch_block(w, generator, emitted.masked)

@@ -382,15 +382,15 @@ class _Small(_SetKernel):
     self.each_part(write)
 
 
-def limit(em):
-  """Largest launch the form is used for. Above one group per CU its groups run one after the
-  other, while the streaming form takes eight per CU at once: with ``r`` rounds of 256 groups it is
-  faster up to 3 for chains of some hundred shared entries, up to 2 for smaller ones (streaming /
+def groups(em):
+  """Most groups per CU of the launches the form is used for. Above one per CU its groups run one
+  after the other, while the streaming form takes eight per CU at once: it is faster up to 3 for
+  chains of some hundred shared entries, up to 2 for smaller ones (streaming /
   this form, volume chains FP64, 9 columns, 2, 3 and 4 rounds: 10 rows, 127 entries 7.0 / 6.3,
   7.6 / 8.0, 8.2 / 9.0 us; 20 rows, 481 entries 11.0 / 8.1, 12.0 / 10.1, 13.0 / 12.0; 35 rows, 1,489
   entries 20.2 / 13.7, 21.3 / 18.7, 22.5 / 23.5; 56 rows, 3,715 entries 33.6 / 19.3, 34.9 / 26.2,
   36.6 / 33.1; FP32, 84 rows, 8,522 entries 52.2 / 25.9, 54.6 / 35.8, 55.1 / 45.3)."""
-  return (3 if em.schedule['shared_entries'] >= 400 else 2) * 256 * em.elements_per_block
+  return 3 if em.schedule['shared_entries'] >= 400 else 2
 
 
 def emit(program, context, base_name, schedule, pl):

@@ -894,7 +894,7 @@ def emit(program, context, base_name, schedule=None) -> Emitted:
       if emitted.lds_bytes <= LDS_LIMIT:
         if schedule.stream_matrix == 'auto':
           emitted.few = small.emit(program, context, base_name, sched, pl)
-          emitted.few_limit = small.limit(emitted.few) if emitted.few else 0
+          emitted.few_groups = small.groups(emitted.few) if emitted.few else 0
         return emitted
   if program.epilogue is not None:
     raise GenerationError('pointwise statements fuse only into a streaming chain')
