@@ -3,21 +3,22 @@ GPU (small time clusters), where the time is that of one wavefront's instruction
 
 The streaming form (:mod:`stream`) gives a wavefront the whole work of its ``64 // q`` elements: 5,400
 instructions for the order-6 volume chain, at two wavefronts per SIMD 18 us whatever the number of
-elements. Here a workgroup of eight wavefronts shares one such group. Its operands come through LDS
+elements. Here a workgroup of four wavefronts shares one such group. Its operands come through LDS
 as in the staged matrix-core form (:mod:`staged`); then
 
-1. each wavefront forms the temporaries ``L_t,e W_t,e`` of an eighth of the contraction rows and
+1. each wavefront forms the temporaries ``L_t,e W_t,e`` of a quarter of the contraction rows and
    leaves them in LDS, one entry per lane;
-2. each wavefront computes an eighth of the destination's rows from all temporaries, one
-   DPP-broadcast FMA per stored entry, in the streaming form's order: the results are the same to
-   the last bit.
+2. each wavefront computes a quarter of the destination's rows from all temporaries, one
+   DPP-broadcast FMA per stored entry, in the streaming form's order: the results of chains that
+   overwrite their destination are the same to the last bit. (One that accumulates adds the old
+   destination at the end here, the streaming form starts from it.)
 
 Order-6 volume chain, streaming form / this one: 100 elements FP64 30.3 / 10.3 us, FP32 25.7 / 8.7;
 1,792 elements (one group on each CU) 32.0 / 12.4 and 26.3 / 9.6. What is left is a chain of
 latencies: the arguments, the loads (one latency for the operands, the shared entries and their
 order), five barriers with an LDS latency each, 1,300 instructions of a wavefront's products at one
-wavefront per SIMD. Eight wavefronts instead of four read every temporary twice as often: the LDS
-bounds (14,336 elements 76 us against 58), 100 elements take the same time.
+wavefront per SIMD. Eight wavefronts were tried: they read every temporary twice as often, which
+the LDS bounds (14,336 elements 76 us against 58), and 100 elements take the same time.
 """
 from dataclasses import replace
 from typing import Optional
@@ -166,9 +167,6 @@ class _Small(_SetKernel):
           ms.append((m, pos))
       out.append(ms)
     return out
-
-  def positions(self, t):
-    return [p for ms in self.columns(t) for _, p in ms]
 
   # ------------------------------------------------------------------ emission
   def emit(self) -> Optional[Emitted]:
