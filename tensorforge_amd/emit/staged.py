@@ -738,12 +738,12 @@ class _Staged(_SetKernel, _Tile):
         self.compute_share(pi)
 
   def compute_share(self, pi):
-    """The wavefront's blocks of the last quantity's contraction, every fourth one."""
+    """The wavefront's blocks of the last quantity's contraction, every fourth one (fused chains)."""
     w, real, ph = self.w, self.real, self.phases[pi]
     x, c = self.xstage[pi], self.q - 1
     welem, wst = self.wstage[pi]
     keys = self.keys(ph)
-    col0 = ph.cols[0] if ph.cols is not None else 0
+    col0 = ph.cols[0]
     w(f'const {real}* __restrict__ xb = lds + {x.lds_base} + el * {x.lds_elem};')
     w(f'const {real}* __restrict__ wb = lds + {self.wbase0} + el * {welem};')
     offs = {ti: off - lo for ti, lo, off, _ in wst}
@@ -760,16 +760,16 @@ class _Staged(_SetKernel, _Tile):
         ops = []
         for j in range(n):
           t, first = self.fresh('xt'), True
-          for m, p in self.slots(ti) if self.fused else ():
+          for m, p in self.slots(ti):
             if p[c] < 0:
               continue
             v, u = f'wb[{offs[ti] + p[c]}]', f'u{keys.index(m)}[{j}]'
             w(f'{real} {t} = {u} * {v};' if first else f'{t} = {self.fp.fma()}({u}, {v}, {t});')
             first = False
           if first:
-            w(f'{real} {t} = {f"({real})0" if self.fused else f"u0[{j}]"};')
+            w(f'{real} {t} = ({real})0;')
           lim = s.krange[1] - s.k0
-          if self.fused and lim < 4 * ph.kr.steps:
+          if lim < 4 * ph.kr.steps:
             # rows past this term's own range must not reach the product
             w(f'{t} = {base} + {j} + {n} * g < {lim} ? {t} : ({real})0;')
           ops.append(t)
