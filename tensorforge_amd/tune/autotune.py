@@ -6,10 +6,14 @@
 * ``method='pick'``: the cost model's choice, nothing timed (the model's mean prediction of
   eight networks trained on the committed MI355X timing database, ``data/timings_mi355x.jsonl.gz``,
   in the project's HIP kernels; trained once per process and device);
-* ``method='pruned'``: the ``k - 1`` best-predicted candidates plus the library's default choice
-  are compiled and timed, the fastest kept;
-* ``method='exhaustive'``: every candidate is compiled and timed (the sweep; the fallback and the
-  yardstick of the other two).
+* ``method='pruned'``: the ``k - 1`` best-predicted candidates plus the kernel the library takes
+  without a schedule are compiled and timed, the fastest kept;
+* ``method='exhaustive'``: every candidate and that kernel are compiled and timed (the sweep; the
+  fallback and the yardstick of the other two).
+
+Where the library's kernel is none of the candidates (matrix-core forms of dense chains, the kernel
+for few elements beside the vector stream, FP32 contraction blocks) it has the label ``default`` and
+the prediction of the vector schedule the model knows as the default; it is never picked untimed.
 
 Forms outside the database the model was trained on (``EXTRA``: the FP64 matrix-core form, for
 FP64 chains with dense shared operands) are never picked by the model; the timed methods time
@@ -91,6 +95,24 @@ def candidates(descrs, fp_type, batch, name_prefix):
   return cands + extra, recs
 
 
+def default_form(descrs, fp_type, cands, name_prefix):
+  """(Candidate, Generator) of the kernel the library takes without a schedule: one of ``cands``
+  where they hold it, else its own, labelled ``default``."""
+  from ..common.context import Context
+  from ..generators.generator import Generator
+  g = Generator(descrs, Context('gfx950', 'hip', fp_type))
+  g.set_kernel_name(f'{name_prefix}_default')
+  g.generate()
+
+  def body(x):
+    lines = x.get_kernel().replace(x.get_emitted().kernel_name, '@').split('\n')
+    return [line for line in lines if not line.lstrip().startswith('//')]
+  for c, other in cands:
+    if body(other) == body(g):
+      return c, other
+  return space.Candidate('default', 'auto', None), g
+
+
 def _prefix(descrs, fp_type, batch):
   """A kernel-name prefix per (chain, type, batch): candidates of different chains loaded into one
   process never share a symbol. The chain's kernel name alone does not separate chains that
@@ -120,8 +142,14 @@ def library(cands, build_dir, force=False):
 def prepare(descrs, fp_type, batch, build_dir, force=False):
   """Compile every candidate of the chain into ``build_dir`` (no GPU needed; an existing object
   is kept unless ``force``); returns the object's path."""
-  cands, _ = candidates(descrs, fp_type, batch, _prefix(descrs, fp_type, batch))
-  return library(cands, build_dir, force)
+  prefix = _prefix(descrs, fp_type, batch)
+  cands, _ = candidates(descrs, fp_type, batch, prefix)
+  return library(_with_default(cands, default_form(descrs, fp_type, cands, prefix)), build_dir,
+                 force)
+
+
+def _with_default(cands, default):
+  return cands if any(g is default[1] for _, g in cands) else cands + [default]
 
 
 def _time(cands, idx, batch, build_dir, device, steps):
@@ -146,7 +174,8 @@ def autotune(descrs, fp_type=FloatingPointType.DOUBLE, batch=65536, method='pick
   """The chosen form of ``descrs`` at ``batch`` elements (see the module docstring)."""
   if method not in ('pick', 'pruned', 'exhaustive'):
     raise ValueError(f'unknown method {method!r}')
-  cands, recs = candidates(descrs, fp_type, batch, _prefix(descrs, fp_type, batch))
+  prefix = _prefix(descrs, fp_type, batch)
+  cands, recs = candidates(descrs, fp_type, batch, prefix)
   labels = [r['label'] for r in recs]
   pred = cost_model(device).predict(M.feature_matrix(recs))
   predicted = dict(zip(labels, (float(p) for p in pred)))
@@ -156,8 +185,16 @@ def autotune(descrs, fp_type=FloatingPointType.DOUBLE, batch=65536, method='pick
     return Choice(labels[i], cands[i][0], cands[i][1], method, predicted)
   if build_dir is None:
     raise ValueError('the timed methods need build_dir for the compiled candidates')
+  default = default_form(descrs, fp_type, cands, prefix)
+  predicted.setdefault(default[0].label, predicted[M.default_choice(labels)])
   extra = list(range(len(recs), len(cands)))
-  idx = M.pruned(order, labels, k) + extra if method == 'pruned' else list(range(len(cands)))
+  cands = _with_default(cands, default)
+  idx = list(range(len(cands)))
+  if method == 'pruned':
+    picks = [int(i) for i in order[:max(1, k - 1)]]
+    picks += [i for i in idx if cands[i][1] is default[1] and i not in picks]
+    picks += [int(i) for i in order if int(i) not in picks][:max(0, k - len(picks))]
+    idx = picks + [i for i in extra if i not in picks]
   timed = _time(cands, idx, batch, build_dir, device, steps)
   best = min(timed, key=timed.get)
   i = [c.label for c, _ in cands].index(best)
