@@ -1,9 +1,9 @@
 """Vector form for few elements: chains with sparse shared operands whose launch does not fill the
 GPU (small time clusters), where the time is that of one wavefront's instructions.
 
-The streaming form (:mod:`stream`) gives a wavefront the whole work of its ``64 // q`` elements: 5,400
-instructions for the order-6 volume chain, at two wavefronts per SIMD 18 us whatever the number of
-elements. Here a workgroup of four wavefronts shares one such group. Its operands come through LDS
+The streaming form (:mod:`stream`) gives a wavefront the whole work of its ``64 // q`` elements:
+5,400 instructions for the order-6 volume chain, at two wavefronts per SIMD 18 us whatever the number
+of elements. Here a workgroup of four wavefronts shares one such group. Its operands come through LDS
 as in the staged matrix-core form (:mod:`staged`); then
 
 1. each wavefront forms the temporaries ``L_t,e W_t,e`` of a quarter of the contraction rows and

@@ -24,12 +24,13 @@ at a time:
 Loads are issued without branches around them and waited for before the results are stored: a
 register written on two paths is copied where they meet, and the memory counter is in order, so
 either mistake turns the requests of the next set into waits (flux integral 428 us with both, 337
-without; derivative step 659 us with 21 spilled registers, 576 with none). Measured, vector form before / this form: C += A B, 56 x 56 by 56 x 9, 65,536 elements FP64
-208 / 138 us (5.7 TB/s); local flux integral, 131,072 elements 468 / 329 us (5.0 TB/s, which is what a
-plain copy of 56 of every 64 rows reaches); neighbour flux integral, 40,001 elements with a mask
-124 / 115 us; time-derivative step, 131,071 elements 618 / 543 us, three arrays, 50,000 elements
-293 / 249 us (both bound by the steps between the barriers of a set: two wavefronts per SIMD do not
-cover their LDS latencies).
+without; derivative step 659 us with 21 spilled registers, 576 with none). Measured, vector form
+before / this form: C += A B, 56 x 56 by 56 x 9, 65,536 elements FP64 208 / 138-142 us (5.6-5.7 TB/s);
+local flux integral, 131,072 elements 468 / 331 us (5.0 TB/s, which is what a plain copy of 56 of
+every 64 rows reaches); neighbour flux integral, 40,001 elements, every fourth masked 124 / 99-102 us
+(116 with the masked ones moved and multiplied); time-derivative step, 131,071 elements
+618 / 541-553 us, three arrays, 50,000 elements 293 / 250-254 us (both bound by the steps between the
+barriers of a set: two wavefronts per SIMD do not cover their LDS latencies).
 """
 from typing import Optional
 
