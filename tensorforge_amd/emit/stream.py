@@ -632,12 +632,12 @@ class _Stream:
     memory or hold many weights in FP64 pay for (800 MB, at the top / early: volume chains FP64 of
     12 rows 230 / 241 us, 35 rows 261 / 273, 64 rows 255 / 248, 84 rows 319 / 310, 56 rows with 27
     weights a column 262 / 295; FP32 35 rows 270 / 284, 56 rows 283 / 273, 20 rows with 27 weights
-    a column 228 / 212)."""
+    a column 228 / 212, 30 rows with 18 weights 267 / 268)."""
     if not self.slots or self.loop or self.dma or \
         any(t.W.arg.addressing != Addressing.STRIDED for t in self.pl.terms if t.kind == 'fused'):
       return False
     held = sum(map(len, self.slots.values()))
-    if self.fp == FloatingPointType.FLOAT and held >= 16:
+    if self.fp == FloatingPointType.FLOAT and held >= 24:
       return True
     return self.busy() and held * self.fp.size() // 4 <= 32
 

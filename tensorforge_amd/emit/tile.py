@@ -958,17 +958,22 @@ def forms(program, pl):
   whole lines (16 x 16 FP64, one column: 99 / 84; 32 x 32 FP32, two columns: 100 / 86), but not for
   shorter ones (4 to 12 rows, two columns: 77-91 / 90-105).
 
-  Flux chains: 32 KB sets 103 direct / 80 staged, 22 KB FP32 99 vector / 91 staged, 16 KB 98 / 99.
-  A chain of one shared operand per term is staged where memory time is as long as matrix time (35
+  Flux chains FP32: 22 KB sets 99 vector / 91 staged, 16 KB 98 / 99; FP64 from 64 KB (44 KB 87 direct /
+  86 staged, but 22 / 26 at 30,000 elements, where the direct form has four sets per workgroup). A
+  chain of one shared operand per term is staged where memory time is as long as matrix time (35
   rows 171 direct / 160 staged, 40 rows 156 / 158), a set has 64 KB (55 KB 113 / 116) and its
   wavefronts form little more than the stored products: one quantity each and a share of a ninth
   (16 columns, 10 rows: 138 vector / 123 direct / 194 staged), with about as many weights in every
   column (28 rows, at most 5 weights in a column, 2.7 on average: 136 / 114 / 158; 3 in every
   column: 137 / 131 / 116).
 
-  The direct form of a chain needs blocks of rows to work on: FP32 blocks have 16 rows (14 rows 127
-  vector / 134 direct, 16 rows 129 / 111, flux chain 10 x 6 rows, three columns 87 / 141), FP64
-  ones 8 (4 rows, one column 79 / 98, nine columns 117 / 113; 6 rows 117 / 109). Of flux chains it
+  The direct form of a chain needs blocks of rows to work on. FP32 blocks have 16 rows (14 rows 127
+  vector / 134 direct, 16 rows 129 / 111, flux chain 10 x 6 rows, three columns 87 / 141); with whole
+  steps of 4 rows it is also faster than a vector form that selects many weights per lane (4 rows, 27
+  weights 117 / 105, 9 weights 143 / 172), and from 13 columns on, where a wavefront of the vector form
+  has four elements or fewer (8 rows, 16 columns 154 / 117, 14 rows, 13 columns 139 / 124 and with 100
+  elements 14.7 / 10.8; 10 rows, 16 columns 152 / 187 and 16.9 / 12.3, 12 columns 107 / 199). FP64 blocks have 8 (6 rows
+  117 / 109; 4 rows, 27 weights 119 / 87, 15 116 / 118, 12 92 / 100, 3 79 / 98). Of flux chains it
   holds two products' accumulators (56 x 21 rows FP64, 10 columns 111 / 109, 13 columns 118 / 129,
   16 columns 127 / 193)."""
   per_set = element_traffic(program).per_element * SET
@@ -981,14 +986,19 @@ def forms(program, pl):
     if per_set >= (13.5 if column >= 112 else 17 if column >= 64 else 32) * 1024:
       return ['staged', 'direct']
     return ['direct'] if few * size >= 128 else []
-  whole = few >= 16 if size == 4 else few >= 6 or per_set >= 16 * 1024
   if pl.post:
-    return ['staged'] * (per_set >= 20 * 1024) + ['direct'] * (whole and pl.q <= WAVES + 1)
+    staged = per_set >= (20 if size == 4 else 64) * 1024
+    whole = few >= 16 if size == 4 else few >= 6 or per_set >= 16 * 1024
+    return ['staged'] * staged + ['direct'] * (whole and pl.q <= WAVES + 1)
   memory, matrix = set_times(program, pl)
   stored = [[len(ms) for _, ms in term_weights(t, range(pl.q))] for t in pl.terms]
-  padded = sum(max(n) * pl.q for n in stored)
+  held = sum(map(max, stored))
   staged = memory >= 0.95 * matrix and per_set >= 64 * 1024 and pl.q <= WAVES + 1 and \
-      padded <= 1.2 * sum(map(sum, stored))
+      held * pl.q <= 1.2 * sum(map(sum, stored))
+  if size == 4:
+    whole = few >= 16 or pl.q >= 13 or (held >= 16 and few % 4 == 0)
+  else:
+    whole = few >= 6 or held >= 15
   return ['staged'] * staged + ['direct'] * whole
 
 

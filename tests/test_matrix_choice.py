@@ -40,10 +40,37 @@ def test_volume(fp, b, form):
   assert _form(w.descrs, fp) == form
 
 
+@pytest.mark.parametrize('fp, b, q, dense, form', [
+  (F64, 4, 9, False, 'vector'), (F64, 4, 16, False, 'direct'), (F64, 6, 9, False, 'direct'),
+  (F32, 8, 9, False, 'vector'), (F32, 8, 16, False, 'direct'), (F32, 10, 12, False, 'vector'),
+  (F32, 10, 13, False, 'direct'), (F32, 4, 9, True, 'direct'), (F32, 10, 9, True, 'vector'),
+  (F32, 16, 9, False, 'direct'), (F64, 10, 16, False, 'direct'), (F64, 40, 9, False, 'direct'),
+  (F64, 35, 9, True, 'staged')])
+def test_volume_by_weights(fp, b, q, dense, form):
+  """Three terms whose columns have the same number of weights."""
+  from tensorforge_amd.common.aux import generate_tmp_tensor
+  from tensorforge_amd.common.basic_types import Addressing
+  from tensorforge_amd.common.matrix.spp import ListSPP
+  from tensorforge_amd.common.matrix.tensor import SubTensor, Tensor
+  from tensorforge_amd.generators.descriptions import MultilinearDescr
+  pair, ident = [[0, -1], [-1, 1]], [[0, 1], [0, 1]]
+  Q, D = (Tensor([b, q], Addressing.STRIDED, alias=x) for x in 'QD')
+  star = None if dense else ListSPP([(r, c) for c in range(q) for r in range(q)
+                                     if (r + 2 * c) % 3 == 0], (q, q))
+  descrs = []
+  for i in range(3):
+    S = Tensor([q, q], Addressing.STRIDED, spp=star, alias=f'S{i}')
+    K = Tensor([b, b], Addressing.NONE, alias=f'K{i}')
+    T = generate_tmp_tensor([SubTensor(Q), SubTensor(S)], pair)
+    descrs += [MultilinearDescr(SubTensor(T), [SubTensor(Q), SubTensor(S)], pair, ident),
+               MultilinearDescr(SubTensor(D), [SubTensor(K), SubTensor(T)], pair, ident, add=i > 0)]
+  assert _form(descrs, fp) == form
+
+
 @pytest.mark.parametrize('fp, m, mid, q, dense, form', [
   (F64, 56, 21, 9, True, 'staged'), (F32, 10, 6, 3, False, 'vector'),
   (F32, 10, 6, 9, True, 'staged'), (F64, 56, 21, 13, False, 'vector'),
-  (F64, 10, 6, 3, False, 'direct')])
+  (F64, 10, 6, 3, False, 'direct'), (F64, 10, 6, 9, True, 'direct')])
 def test_flux(fp, m, mid, q, dense, form):
   e = catalog._matrix_entry('chain', m=m, mid=mid, k=m, q=q, fp=fp, beta=1.0, dense_star=dense)
   assert _form(e.descrs, fp) == form
